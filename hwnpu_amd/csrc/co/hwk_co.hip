@@ -123,7 +123,10 @@ __device__ __forceinline__ void co_gemm(const uint32_t *X, const uint8_t *W, con
     return;
   }
   const bool equads = MX && (k / 32) % 16 == 0 && ((uintptr_t)E & 15) == 0;
-  hwk_gemm::gemm_wg<128, 128, MX, 2, 2>(blockIdx.x, (const u32x4 *)X, W, E, S, Y, m, n, k, (int)mode, equads);
+  // the library's k groups for the shape, so that the sums are its own bit for bit
+  const uint32_t groups = hwk_gemm::pair_takes(MX, m, n, k, E) ? hwk_gemm::pair_groups(MX, m, n, k) : 1;
+  hwk_gemm::gemm_wg<128, 128, MX, 2, 2, 1, true>(blockIdx.x, (const u32x4 *)X, W, E, S, Y, m, n, k, (int)mode, equads,
+                                                 groups);
 }
 
 __device__ __forceinline__ hwk_moe::MoeArgs moe_args(uint32_t T, uint32_t H, uint32_t I, uint32_t E, uint32_t k,

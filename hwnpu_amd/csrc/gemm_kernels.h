@@ -2,20 +2,16 @@
 // kernels of the library's code object (co/hwk_co.hip), so that both run the same instructions.
 //
 // Prefill / verify GEMM (K3) on gfx950: Y (M, N) = X (M, K) W^T, X fp16, W int8 per output channel
-// or MXFP4, fp32 accumulation on the fp16 MFMA (v_mfma_f32_16x16x32_f16).
+// or MXFP4, fp32 accumulation on the fp16 MFMA (v_mfma_f32_16x16x32_f16). Weights are converted next to
+// the MFMAs that take them: int8 exactly to fp16 (the channel scale applied to the fp32 result), MXFP4 by
+// the hardware fp4 conversion with the block scale folded in.
 //
-// A workgroup of 4 waves (one a SIMD, 2 x 2) computes a BM x BN tile of Y; a wave holds a
-// (BM/2) x (BN/2) block of 16 x 16 accumulator tiles. K goes 128 at a time:
-//   X: the tile's 128-column slab goes through LDS (two buffers, one barrier a step), 16-byte chunks
-//      placed at chunk ^ (row & 15) so that the 16 rows one MFMA operand load touches fall in 16
-//      different bank groups (a row is 256 bytes, the width of the 64 banks);
-//   W: each wave loads its own columns' codes straight into registers (16 or 32 bytes a lane per 16
-//      columns a step) and converts them there: int8 exactly to fp16 (the channel scale applied to
-//      the fp32 result), MXFP4 by the hardware fp4 conversion with the block scale folded in.
-// Loads run two steps ahead of the multiply (register stages), so a step's global latency hides
-// behind the two steps before it. A lane's 32 values of K a step are the same set in its X and W
-// operands, so each MFMA sums 32 true products (which lane holds which k is a free choice of the
-// kernel, made for contiguous loads).
+// Two forms. The paired form (gemm_pair_wg, K a multiple of 64) takes nearly everything: operands straight
+// from memory into LDS rings, one barrier a step of 64 values, tiles from 16 x 32 to 128 x 256 and, for tiles
+// that would leave CUs or waves idle, several k groups of waves a workgroup (pick_pair chooses). The general
+// form (gemm_wg) takes any K that is a multiple of 32, operands past 4 GiB and odd scale addresses: a
+// BM x BN tile, K 128 at a time with X through LDS (two buffers, one barrier a step) and the weights loaded
+// into registers two steps ahead.
 //
 // MXFP4 exactness: a code times its block scale is an fp16 value when the scale's exponent is in
 // [-23, 13]. A row (output channel) whose finite block exponents leave that range is shifted by a
@@ -23,10 +19,9 @@
 // by 2^s0, which is exact; rows whose exponents span more than 36 lose the low bits of their
 // smallest blocks (values below 2^-24 of the shifted scale). Scale e = 0 is 0 and e = 255 is +Inf,
 // as in the reference's Dequantize (internal/mxfp4/mxfp4.go:77).
-//
-// Tile order is XCD-aware: the workgroups that share a weight panel run on the same XCD, so its L2
-// holds the panel once; the host picks the tile shape that fills the 256 CUs best.
 #pragma once
+
+#include <type_traits>
 
 #include "hwk_common.h"
 
@@ -70,12 +65,14 @@ __device__ __forceinline__ half8 fp4x8_to_half8(uint32_t w, float s) {
 __device__ __forceinline__ u32x4 load16(const void *p) { return *(const u32x4 *)p; }
 
 // The X chunk (of CH a row a step) that MFMA kk of lane group q reads: the k offsets of a lane's
-// operands in the step. int8: two 16-byte weight loads a lane at q*16 and 64 + q*16 (each 16 rows x 64
-// contiguous bytes a load instruction); MXFP4: one 32-value block a lane at q*32.
-template <bool MX>
-__device__ __forceinline__ int xchunk(int q, int kk) {
-  if constexpr (MX) return 4 * q + kk;
-  return kk < 2 ? 2 * q + kk : 8 + 2 * q + (kk - 2);
+// operands in the step. A lane takes 16 values in a row of each 64: values q*16 .. +15 (MFMAs 0, 1) and
+// 64 + q*16 .. +15 (MFMAs 2, 3), of int8 and MXFP4 weights alike. Every form of the GEMM feeds its MFMAs
+// these sets in this order, so that forms and tile shapes agree bit for bit (given the same segments of K).
+__device__ __forceinline__ int xchunk(int q, int kk) { return kk < 2 ? 2 * q + kk : 8 + 2 * q + (kk - 2); }
+
+// The first 128-value step of segment g when the S steps of K go to KG segments.
+__host__ __device__ __forceinline__ uint32_t seg_first(uint32_t S, uint32_t KG, uint32_t g) {
+  return (uint32_t)((uint64_t)g * S / KG);
 }
 
 // KG k groups of WM x WN waves: group g takes MFMAs g*KK/KG .. of every step of the whole tile, and
@@ -96,7 +93,7 @@ template <int BM, int BN, bool MX, int WM, int WN, int KG>
 struct Stage {
   u32x4 a[Cfg<BM, BN, MX, WM, WN, KG>::AL];
   u32x4 b[Cfg<BM, BN, MX, WM, WN, KG>::TN][Cfg<BM, BN, MX, WM, WN, KG>::BL];
-  uint32_t e[Cfg<BM, BN, MX, WM, WN, KG>::TN];  // MXFP4 block scale bytes
+  uint32_t e[Cfg<BM, BN, MX, WM, WN, KG>::TN][2];  // MXFP4: the scale bytes of the lane's two blocks
   uint32_t k0;                                  // the step's K offset
 };
 
@@ -125,12 +122,16 @@ __device__ __forceinline__ void load_w(Stage<BM, BN, MX, WM, WN, KG> &s, const u
                                        const uint32_t (&brow)[Cfg<BM, BN, MX, WM, WN, KG>::TN], int q, int g) {
   using C = Cfg<BM, BN, MX, WM, WN, KG>;
   if constexpr (MX) {
-    const uint32_t blk = min(k0 + q * 32, K - 32) / 32;
 #pragma unroll
-    for (int j = 0; j < C::TN; j++) {
-      const size_t bi = (size_t)brow[j] * (K / 32) + blk;
-      s.b[j][0] = load16(W + bi * 16);
-      s.e[j] = E[bi];
+    for (int h = 0; h < 2; h++) {
+      const uint32_t kc = min(k0 + h * 64 + q * 16, K - 16);
+#pragma unroll
+      for (int j = 0; j < C::TN; j++) {
+        const u32x2 v = *(const u32x2 *)(W + (size_t)brow[j] * (K / 2) + kc / 2);
+        s.b[j][0][2 * h] = v[0];
+        s.b[j][0][2 * h + 1] = v[1];
+        s.e[j][h] = E[(size_t)brow[j] * (K / 32) + kc / 32];
+      }
     }
   } else {
 #pragma unroll
@@ -153,10 +154,12 @@ __device__ __forceinline__ void zero_tail(Stage<BM, BN, MX, WM, WN, KG> &s, uint
 #pragma unroll
   for (int j = 0; j < C::TN; j++) {
     if constexpr (MX) {
-      if (s.k0 + q * 32 >= K) {
-        s.b[j][0] = zero;
-        s.e[j] = 0u;
-      }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        if (s.k0 + h * 64 + q * 16 >= K) {
+          s.b[j][0][2 * h] = s.b[j][0][2 * h + 1] = 0u;
+          s.e[j][h] = 0u;
+        }
     } else {
 #pragma unroll
       for (int h = 0; h < C::BL; h++)
@@ -241,10 +244,12 @@ __device__ __forceinline__ void tile_of(uint32_t id, uint32_t mt, uint32_t nt, u
 
 // The tile's store: D of MFMA tile (i, j) of the wave, lane (r16, q) holding rows q*4 + r of column
 // r16; int8 results take the column's scale, MXFP4 results the row shift back (2^s0, exact).
-template <int BM, int WM, int TM, int TN, bool MX>
+// KG > 1: the 16-row tiles i = own, own + KG, ... only.
+template <int BM, int WM, int TM, int TN, bool MX, int KG = 1>
 __device__ __forceinline__ void store_tile(const floatx4 (&acc)[TM][TN], const int (&s0)[TN],
                                            const uint16_t *__restrict__ S, void *__restrict__ Y, uint32_t M,
-                                           uint32_t N, uint32_t m0, uint32_t nw, int wm, int r16, int q, int mode) {
+                                           uint32_t N, uint32_t m0, uint32_t nw, int wm, int r16, int q, int mode,
+                                           int own = 0) {
   if (mode == kOutSwiGLU) {
     // columns (2c, 2c+1) are (gate, up) of output c, held by lanes r16 and r16 ^ 1 for the same four
     // rows: the gate lane takes the up values of rows 0, 1 and computes those outputs, the up lane
@@ -257,6 +262,7 @@ __device__ __forceinline__ void store_tile(const floatx4 (&acc)[TM][TN], const i
       const float sc = MX ? 1.0f : (float)__builtin_bit_cast(f16, S[min(n, N - 1)]);
 #pragma unroll
       for (int i = 0; i < TM; i++) {
+        if (KG > 1 && i % KG != own) continue;
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) v[r] = MX ? ldexpf(acc[i][j][r], s0[j]) : acc[i][j][r] * sc;
@@ -276,113 +282,114 @@ __device__ __forceinline__ void store_tile(const floatx4 (&acc)[TM][TN], const i
     if (n >= N) continue;
     const float sc = MX ? 1.0f : (float)__builtin_bit_cast(f16, S[n]);
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+    for (int i = 0; i < TM; i++) {
+      if (KG > 1 && i % KG != own) continue;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const uint32_t m = m0 + wm * (BM / WM) + i * 16 + q * 4 + r;
         if (m < M) store_out(Y, (size_t)m * N + n, MX ? ldexpf(acc[i][j][r], s0[j]) : acc[i][j][r] * sc, mode);
       }
+    }
   }
 }
 
-// The same stores through LDS: the wave's block (RW x CW) into its region st of LDS, as the values
-// stored (fp16 rounded, or SwiGLU'd pairs, or scaled fp32), then 16-byte pieces of its rows to Y: an
-// MFMA tile's lanes hold one column each, so a direct store instruction writes 2 or 4 bytes a lane.
-// Every value is rounded and combined as store_tile does it. The fp32 rows are padded (P32 = CW + 4
-// floats) so that the 4 row groups of a write land in different banks (P32 = CW where the padded
-// block does not fit); the fp16 rows are not (padding them measured no faster: their reads of 16
-// bytes a lane then conflict). Needs Y 16-byte aligned and N a multiple of the piece (4 fp32, 8 fp16
-// or 16 SwiGLU columns): staged() tells.
+// LDS writes and reads of this wave done (lgkmcnt 0; the other counters not waited for)
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
+
+// The tile's store through LDS, 16 rows of the wave's block at a time (a strip): the values as stored
+// (fp16 rounded, SwiGLU'd pairs, or scaled fp32), then 16-byte pieces of the rows to Y, since an MFMA
+// tile's lanes hold one column each. Every value is rounded and combined as store_tile does it. st: the
+// wave's 16 x (TN*16 + 4) floats of LDS. For staged(Y, N, mode).
 __device__ __forceinline__ bool staged(const void *Y, uint32_t N, int mode) {
   const uint32_t piece = mode == kOutSwiGLU ? 16 : mode == HWK_OUT_F16 ? 8 : 4;
   return ((uintptr_t)Y & 15) == 0 && N % piece == 0;
 }
-template <int TM, int TN, int P32>
-struct StageRows {
-  static constexpr int RW = TM * 16, CW = TN * 16;
-  static constexpr int P16 = CW, PH = CW / 2 + 8;  // fp16 rows: full width, SwiGLU half width (padded)
-  static constexpr int FLOATS = RW * P32;              // a region, in floats (the largest of the three)
-  static_assert(P32 == CW || P32 == CW + 4, "fp32 row stride");
-  static_assert(RW * P16 * 2 <= FLOATS * 4 && RW * PH * 2 <= FLOATS * 4, "fp16 rows fit the region");
-};
-template <int BM, int WM, int TM, int TN, bool MX, int P32>
-__device__ __forceinline__ void store_tile_staged(const floatx4 (&acc)[TM][TN], const int (&s0)[TN],
-                                                  const uint16_t *__restrict__ S, void *__restrict__ Y, uint32_t M,
-                                                  uint32_t N, uint32_t m0, uint32_t nw, int wm, int lane, int mode,
-                                                  float *st) {
-  using G = StageRows<TM, TN, P32>;
-  constexpr int RW = G::RW, CW = G::CW;
+// KG > 1: strips own, own + KG, ... only.
+template <int TM, int TN, bool MX, int KG = 1>
+__device__ __forceinline__ void store_strips(const floatx4 (&acc)[TM][TN], const int (&s0)[TN], bool shift,
+                                             const uint16_t *__restrict__ S, void *__restrict__ Y, uint32_t M,
+                                             uint32_t N, uint32_t r0, uint32_t nw, int lane, int mode, float *st,
+                                             int own = 0) {
+  constexpr int CW = TN * 16, P32 = CW + 4, P16 = CW + 8, PH = CW / 2 + 8;
   const int r16 = lane & 15, q = lane >> 4;
-  const uint32_t r0 = m0 + wm * RW;
+  float sc[TN];
+#pragma unroll
+  for (int j = 0; j < TN; j++) sc[j] = MX ? 1.0f : (float)__builtin_bit_cast(f16, S[min(nw + j * 16 + r16, N - 1)]);
   auto value = [&](int i, int j, int r) __attribute__((always_inline)) {
-    const float sc = MX ? 1.0f : (float)__builtin_bit_cast(f16, S[min(nw + j * 16 + r16, N - 1)]);
-    return MX ? ldexpf(acc[i][j][r], s0[j]) : acc[i][j][r] * sc;
+    if constexpr (MX) return shift ? ldexpf(acc[i][j][r], s0[j]) : acc[i][j][r];
+    else return acc[i][j][r] * sc[j];
   };
+  f16 *h = (f16 *)st;
   if (mode == kOutSwiGLU) {
     // the pairs as store_tile makes them: gate lane rows 0, 1 of its quad, up lane rows 2, 3
-    f16 *h = (f16 *)st;
     const bool gate = (r16 & 1) == 0;
 #pragma unroll
-    for (int j = 0; j < TN; j++)
+    for (int i = 0; i < TM; i++) {
+      if (KG > 1 && i % KG != own) continue;
 #pragma unroll
-      for (int i = 0; i < TM; i++) {
+      for (int j = 0; j < TN; j++) {
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) v[r] = value(i, j, r);
         const float o0 = __shfl_xor(gate ? v[2] : v[0], 1, 64), o1 = __shfl_xor(gate ? v[3] : v[1], 1, 64);
-        const int row = i * 16 + q * 4 + (gate ? 0 : 2), c = (j * 16 + r16) / 2;
-        h[row * G::PH + c] = (f16)(gate ? swiglu_value(v[0], o0) : swiglu_value(o0, v[2]));
-        h[(row + 1) * G::PH + c] = (f16)(gate ? swiglu_value(v[1], o1) : swiglu_value(o1, v[3]));
+        const int row = q * 4 + (gate ? 0 : 2), c = (j * 16 + r16) / 2;
+        h[row * PH + c] = (f16)swiglu_value(gate ? v[0] : o0, gate ? o0 : v[2]);
+        h[(row + 1) * PH + c] = (f16)swiglu_value(gate ? v[1] : o1, gate ? o1 : v[3]);
       }
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // this wave's LDS writes done
-    constexpr int CPR = CW / 16;  // 8 outputs a piece
-    for (int c = lane; c < RW * CPR; c += 64) {
-      const int row = c / CPR, k = c % CPR;
-      const uint32_t m = r0 + row, n = nw + k * 16;
-      if (m < M && n < N)
-        *(u32x4 *)((f16 *)Y + (size_t)m * (N / 2) + n / 2) = *(const u32x4 *)(h + row * G::PH + k * 8);
+      wait_lds();
+      constexpr int CPR = CW / 16;  // pieces of 8 outputs a row
+      for (int c = lane; c < 16 * CPR; c += 64) {
+        const int row = c / CPR, k = c % CPR;
+        const uint32_t m = r0 + i * 16 + row, n = nw + k * 16;
+        if (m < M && n < N) *(u32x4 *)((f16 *)Y + (size_t)m * (N / 2) + n / 2) = *(const u32x4 *)(h + row * PH + k * 8);
+      }
     }
   } else if (mode == HWK_OUT_F16) {
-    f16 *h = (f16 *)st;
 #pragma unroll
-    for (int j = 0; j < TN; j++)
+    for (int i = 0; i < TM; i++) {
+      if (KG > 1 && i % KG != own) continue;
 #pragma unroll
-      for (int i = 0; i < TM; i++)
+      for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) h[(i * 16 + q * 4 + r) * G::P16 + j * 16 + r16] = (f16)f32_value(value(i, j, r));
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
-    constexpr int CPR = CW / 8;
-    for (int c = lane; c < RW * CPR; c += 64) {
-      const int row = c / CPR, k = c % CPR;
-      const uint32_t m = r0 + row, n = nw + k * 8;
-      if (m < M && n < N) *(u32x4 *)((f16 *)Y + (size_t)m * N + n) = *(const u32x4 *)(h + row * G::P16 + k * 8);
+        for (int r = 0; r < 4; r++) h[(q * 4 + r) * P16 + j * 16 + r16] = (f16)f32_value(value(i, j, r));
+      wait_lds();
+      constexpr int CPR = CW / 8;
+      for (int c = lane; c < 16 * CPR; c += 64) {
+        const int row = c / CPR, k = c % CPR;
+        const uint32_t m = r0 + i * 16 + row, n = nw + k * 8;
+        if (m < M && n < N) *(u32x4 *)((f16 *)Y + (size_t)m * N + n) = *(const u32x4 *)(h + row * P16 + k * 8);
+      }
     }
   } else {
 #pragma unroll
-    for (int j = 0; j < TN; j++)
+    for (int i = 0; i < TM; i++) {
+      if (KG > 1 && i % KG != own) continue;
 #pragma unroll
-      for (int i = 0; i < TM; i++)
+      for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) st[(i * 16 + q * 4 + r) * P32 + j * 16 + r16] = value(i, j, r);
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
-    constexpr int CPR = CW / 4;
-    for (int c = lane; c < RW * CPR; c += 64) {
-      const int row = c / CPR, k = c % CPR;
-      const uint32_t m = r0 + row, n = nw + k * 4;
-      if (m >= M || n >= N) continue;
-      floatx4 v = *(const floatx4 *)(st + row * P32 + k * 4);
-      floatx4 *y = (floatx4 *)((float *)Y + (size_t)m * N + n);
-      if (mode == HWK_OUT_ADD_F32) v = *y + v;
-      *y = v;
+        for (int r = 0; r < 4; r++) st[(q * 4 + r) * P32 + j * 16 + r16] = value(i, j, r);
+      wait_lds();
+      constexpr int CPR = CW / 4;
+      for (int c = lane; c < 16 * CPR; c += 64) {
+        const int row = c / CPR, k = c % CPR;
+        const uint32_t m = r0 + i * 16 + row, n = nw + k * 4;
+        if (m >= M || n >= N) continue;
+        floatx4 v = *(const floatx4 *)(st + row * P32 + k * 4);
+        floatx4 *y = (floatx4 *)((float *)Y + (size_t)m * N + n);
+        if (mode == HWK_OUT_ADD_F32) v = *y + v;
+        *y = v;
+      }
     }
   }
 }
 
-template <int BM, int BN, bool MX, int WM, int WN, int KG = 1>
+// SEG: the accumulators of nseg segments of K (seg_first) are added in order, as the paired form's k groups'
+// are (one segment: the plain sum).
+template <int BM, int BN, bool MX, int WM, int WN, int KG = 1, bool SEG = false>
 __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X, const uint8_t *__restrict__ W,
                                         const uint8_t *__restrict__ E, const uint16_t *__restrict__ S,
                                         void *__restrict__ Y, uint32_t M, uint32_t N, uint32_t K, int mode,
-                                        bool equads) {
+                                        bool equads, uint32_t nseg = 1) {
   using C = Cfg<BM, BN, MX, WM, WN, KG>;
   constexpr int TM = C::TM, TN = C::TN, NT = C::NT, KKG = C::KKG;
   static_assert(KG == 1 || !MX, "k groups here: int8 only");
@@ -432,6 +439,14 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int j = 0; j < TN; j++) acc[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+  floatx4 total[SEG ? TM : 1][SEG ? TN : 1];
+  uint32_t seg = 0;
+  if constexpr (SEG) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) total[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+  }
 
   // Steps in groups of NS (a partial last group multiplies zeros: its loads read past K). A step:
   // its X slab into LDS, barrier, the next X loads of its stage, then for each kk its weight operands
@@ -453,22 +468,24 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
       issue_order();
       load_x<BM, BN, MX, WM, WN, KG>(st[s], X, M, K, m0, kofs(j + NS), t);
       issue_order();
-      float sc[TN];
+      float sc[TN][2];
 #pragma unroll
-      for (int jn = 0; jn < TN; jn++) sc[jn] = MX ? shifted_scale(st[s].e[jn], s0[jn]) : 0.0f;
+      for (int jn = 0; jn < TN; jn++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) sc[jn][h] = MX ? shifted_scale(st[s].e[jn][h], s0[jn]) : 0.0f;
       // the operands of kk + 1 (X from LDS, weights converted) are fetched before the MFMAs of kk; kk
       // counts the group's MFMAs (the step's MFMA g*KKG + kk)
       auto operands = [&](half8 (&af)[TM], half8 (&bf)[TN], int kk) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < TM; i++) {
           const int row = wm * (BM / WM) + i * 16 + r16;
-          const int ch = KG == 1 ? xchunk<MX>(q, kk) : xchunk<MX>(q, g * KKG + kk);
+          const int ch = KG == 1 ? xchunk(q, kk) : xchunk(q, g * KKG + kk);
           af[i] = __builtin_bit_cast(half8, buf[row * CH + (ch ^ (row & 15))]);
         }
 #pragma unroll
         for (int jn = 0; jn < TN; jn++) {
           if constexpr (MX) {
-            bf[jn] = fp4x8_to_half8(st[s].b[jn][0][kk], sc[jn]);
+            bf[jn] = fp4x8_to_half8(st[s].b[jn][0][kk], sc[jn][kk >> 1]);
           } else {
             const u32x4 v = st[s].b[jn][kk >> 1];  // KG = 2: the group's half, loaded alone
             bf[jn] = i8x8_to_half8(v[(kk & 1) * 2], v[(kk & 1) * 2 + 1]);
@@ -489,7 +506,23 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
       issue_order();
       load_w<BM, BN, MX, WM, WN, KG>(st[s], W, E, K, kofs(j + NS), brow, q, g);
       issue_order();
+      if constexpr (SEG) {
+        for (; seg < nseg && seg_first(steps, nseg, seg + 1) <= j + 1; seg++)  // (empty segments add zeros)
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int jn = 0; jn < TN; jn++) {
+              total[i][jn] += acc[i][jn];
+              acc[i][jn] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+            }
+      }
     }
+  }
+  if constexpr (SEG) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) acc[i][j] = total[i][j];
   }
   if constexpr (KG == 2) {
     // group 1's accumulators to group 0 through the X buffers (every wave is done with them after
@@ -513,346 +546,356 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
     if (g == 1) return;
   }
   if (staged(Y, N, mode)) {
-    // a wave's block in region wl of the X buffers (rows padded where that fits)
-    constexpr int CW = TN * 16, PAD = WM * WN * TM * 16 * (CW + 4) <= 2 * BM * CH * 4 ? CW + 4 : CW;
-    using G = StageRows<TM, TN, PAD>;
-    static_assert(WM * WN * G::FLOATS <= 2 * BM * CH * 4, "the staged blocks fit the X buffers");
+    static_assert(WM * WN * 16 * (TN * 16 + 4) * 4 <= 2 * BM * CH * 16, "the store strips fit the X buffers");
     if constexpr (KG == 1) __syncthreads();  // every wave is done with the X buffers
-    store_tile_staged<BM, WM, TM, TN, MX, PAD>(acc, s0, S, Y, M, N, m0, nw, wm, lane, mode,
-                                               (float *)&As[0][0] + wl * G::FLOATS);
+    store_strips<TM, TN, MX>(acc, s0, true, S, Y, M, N, m0 + wm * (BM / WM), nw, lane, mode,
+                             (float *)&As[0][0] + wl * 16 * (TN * 16 + 4));
     return;
   }
   store_tile<BM, WM, TM, TN, MX>(acc, s0, S, Y, M, N, m0, nw, wm, r16, q, mode);
 }
 
 
-// ---- The ring form (K a multiple of 128): X and the weights both go straight from memory into LDS ----
+// ---- The paired form (K a multiple of 64): two workgroups a CU ----
 //
-// Every global load of the main loop is a load into LDS (global_load_lds_dwordx4: lane i of an
-// instruction writes 16 bytes at the instruction's LDS base + 16 i), into a ring of RS buffers a
-// stream (a template parameter), issued RS-1 steps ahead of the MFMAs that read them, and waited for
-// by an explicit count
-// (the wait counter is in order, and every step issues the same number of loads: past the last step
-// they reread in-range data into a buffer nobody reads). No load result lives in a register across
-// steps, so the loop carries nothing for the compiler to wait on at its head. The swizzles are applied
-// on the source side (which 16-byte chunk a lane fetches), so that the MFMA operand reads of 16
-// lanes land in distinct banks:
-//   X   slot p: row p / CH, chunk (p % CH) ^ (row & 15)                       (256-byte rows)
-//   W   slot p: column p / WCH, chunk (p % WCH) ^ ((column / CPB) & (WCH-1))    (WCH chunks a column a
-//       step: int8 8 = 128 codes, MXFP4 4 = 128 values; CPB columns share a 256-byte bank row)
-//   E   (MXFP4) slot p: column p, the 4 scale bytes of the step (4-byte loads)
-// An LDS buffer of BYTES, one variable per (BYTES, I, TAG): the buffers of a ring are distinct
-// variables, so that the compiler can tell an LDS read of one from the loads into LDS in flight for
-// the others.
-template <typename T, int COUNT, int I, int TAG>
-__device__ __forceinline__ T *lds_buf() {
-  __shared__ __attribute__((aligned(16))) T b[COUNT];
-  return b;
-}
-template <typename T, int COUNT, int TAG, int N>
-struct RingBufs {
-  static __device__ __forceinline__ void fill(T **p) {
-    RingBufs<T, COUNT, TAG, N - 1>::fill(p);
-    p[N - 1] = lds_buf<T, COUNT, N - 1, TAG>();
-  }
-};
-template <typename T, int COUNT, int TAG>
-struct RingBufs<T, COUNT, TAG, 0> {
-  static __device__ __forceinline__ void fill(T **) {}
-};
+// K goes 64 at a time through a ring of three LDS stages, X and the weights straight from memory into LDS
+// (global_load_lds: lane i of an instruction writes 16 bytes at the instruction's LDS base + 16 i), two
+// steps ahead, waited for by an explicit count (the wait counter is in order, and a wave issues the same
+// number of loads every step: past the last step they reread in-range data into a stage nobody reads).
+// A step is one barrier, the operand reads and the MFMAs; nothing is carried in registers but the
+// accumulators, so that a wave fits 128 registers and a CU holds two workgroups: while one waits at its
+// barrier, scans or stores its tile (the SwiGLU's float64 exp), the other's MFMAs run.
+// The swizzles are applied on the source side (which 16-byte chunk a lane fetches), so that the reads of
+// 16 lanes land in distinct banks:
+//   X   slot p: row p / 8, chunk (p % 8) ^ ((row >> 1) & 7)                (128-byte rows)
+//   W   int8   slot p: column p / 4, chunk (p % 4) ^ ((column >> 2) & 3)   (64-byte columns)
+//       MXFP4  slot p: column p / 2, chunk (p % 2) ^ ((column >> 3) & 1)   (32-byte columns)
+//   E   (MXFP4) dword p: column p, the step's two scale bytes
 
-template <int BM, int BN, bool MX, int WM, int WN, int KG, int RS>
-struct RCfg {
-  using C = Cfg<BM, BN, MX, WM, WN, KG>;
-  static constexpr int NT = C::NT, NW = NT / 64;
-  static constexpr int WCH = MX ? 4 : 8;                             // 16-byte weight chunks a column a step
-  static constexpr int CPB = 256 / (WCH * 16);                       // columns a 256-byte bank row
-  static constexpr int AX = BM * CH / NT;                            // X loads a lane a step
-  static constexpr int AW = (BN * WCH + NT - 1) / NT;                // weight loads a lane a step
-  static constexpr int WSLOTS = AW * NT;                             // weight slots a buffer (padded)
-  static constexpr int LS = AX + AW + (MX ? 1 : 0);                  // loads a lane a step (E: one)
-  static_assert(BM * CH % NT == 0, "X loads a lane");
-  static_assert(!MX || BN <= NT, "scale slots");
-  static_assert((RS - 1) * LS <= 63, "loads in flight past the wait counter");
+
+// A tile of the paired form: BM x BN, WM x WN waves a k group, KG k groups, RS ring stages, the workgroups of
+// it that a CU holds (res), and the picoseconds of a CU that the tile takes a value of K (ps).
+struct PairTile {
+  uint16_t bm, bn, wm, wn, kg, rs, res, ps;
 };
+#define HWK_PAIR_MX(F)                                                                                       \
+  F(128, 256, 2, 4, 1, 3, 2, 14261) F(128, 192, 2, 4, 1, 3, 2, 11273) F(128, 128, 2, 2, 2, 3, 1, 8300)       \
+  F(128, 64, 4, 2, 2, 3, 1, 5439) F(96, 64, 2, 2, 2, 3, 1, 4141) F(64, 64, 2, 2, 2, 3, 2, 3048)              \
+  F(32, 64, 2, 2, 4, 4, 1, 2404) F(32, 32, 2, 1, 4, 4, 1, 1350) F(16, 32, 1, 2, 8, 4, 1, 1070)
+#define HWK_PAIR_I8(F)                                                                                       \
+  F(128, 128, 2, 4, 1, 3, 2, 8075) F(128, 128, 2, 4, 2, 3, 1, 8000) F(128, 96, 2, 3, 2, 3, 1, 6578)          \
+  F(128, 64, 4, 2, 2, 3, 1, 5461) F(64, 64, 2, 2, 2, 3, 2, 2854) F(32, 64, 2, 2, 4, 3, 1, 2128)              \
+  F(32, 32, 2, 2, 4, 4, 1, 1391) F(16, 32, 1, 2, 8, 4, 1, 769)
+
+// The tile of least cost for Y (m, n) over k, an index into HWK_PAIR_MX or HWK_PAIR_I8. The cost is that of
+// the busiest of the 256 CUs: ps * k for each of its tiles, and 3.9 us (prologue, the first loads' latency,
+// the groups' sums and the stores) for each round of res tiles. Both constants are fitted to every tile's
+// time on 154 (MXFP4) and 137 (int8) shapes, m 9..8192, n 512..16384, k 512..8192: the tile picked is on
+// average 1 % slower than the best of the table and takes 0.47 (MXFP4) and 0.50 (int8) of the time of the
+// one-workgroup-a-CU tiles of 64..128 rows that stood here before. (int8 128 x 128 in two k groups is set just
+// below the one-group tile, which it beats by 3-7 % when a CU has one tile.) Integer arithmetic, so that
+// the host and a kernel agree.
+__host__ __device__ __forceinline__ int pick_pair(bool mx, uint32_t m, uint32_t n, uint32_t k) {
+#define HWK_TILE(...) {__VA_ARGS__},
+  constexpr PairTile kMx[] = {HWK_PAIR_MX(HWK_TILE)}, kI8[] = {HWK_PAIR_I8(HWK_TILE)};
+#undef HWK_TILE
+  constexpr int kNMx = sizeof kMx / sizeof kMx[0], kNI8 = sizeof kI8 / sizeof kI8[0];
+  int best = 0;
+  uint64_t best_cost = ~0ull;
+  for (int i = 0; i < (mx ? kNMx : kNI8); i++) {
+    const PairTile t = mx ? kMx[i] : kI8[i];
+    const uint64_t tiles = (uint64_t)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+    const uint64_t most = (tiles + 255) / 256;  // tiles of the busiest CU
+    const uint64_t cost = most * t.ps * k + (most + t.res - 1) / t.res * 3900000ull;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = i;
+    }
+  }
+  return best;
+}
+// The k groups of the tile picked.
+__host__ __device__ __forceinline__ uint32_t pair_groups(bool mx, uint32_t m, uint32_t n, uint32_t k) {
+  const int i = pick_pair(mx, m, n, k);
+#define HWK_KG(bm, bn, wm, wn, kg, rs, res, ps) kg,
+  constexpr uint8_t kMx[] = {HWK_PAIR_MX(HWK_KG)}, kI8[] = {HWK_PAIR_I8(HWK_KG)};
+#undef HWK_KG
+  return mx ? kMx[i] : kI8[i];
+}
+// Whether the paired form takes a product: whole steps of 64 values, scale bytes readable two at a time, and
+// its loads' 32-bit byte offsets.
+__host__ __device__ __forceinline__ bool pair_takes(bool mx, uint32_t m, uint32_t n, uint32_t k, const void *e) {
+  return k % 64 == 0 && (!mx || ((uintptr_t)e & 1) == 0) && (uint64_t)m * k * 2 < (1ull << 32) &&
+         (uint64_t)n * (mx ? k / 2 : k) < (1ull << 32);
+}
 
 template <int N>
 __device__ __forceinline__ void wait_loads() {
   static_assert(N >= 0 && N <= 63, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
-// LDS writes and reads of this wave done (lgkmcnt 0; the other counters not waited for)
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
 // A workgroup barrier that waits for no memory counter (__syncthreads would wait for every load into
 // LDS in flight, the ring's prefetches included): the caller has waited for its own part.
 __device__ __forceinline__ void ring_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
 typedef __attribute__((address_space(3))) void lds_void;
-// The loads into LDS as inline assembly, so that the compiler inserts no wait of its own for them: its
+// The loads into LDS as inline assembly, so that the compiler inserts no wait of its own for them (its
 // wait insertion tracks the LDS targets of a few such loads only, and before an LDS read that none of
-// those covers it waits for every load in flight (vmcnt(0): in the software-pipelined loop below,
-// two steps of six drained the prefetch that way). The ring's explicit vmcnt waits and barriers order
-// them instead; the "memory" clobber keeps LDS reads and the barriers on their side of each load.
-// The LDS address (wave-uniform) goes in M0 as an operand the compiler sets, the s_nop the wait state
-// between that write and the load; the global address is sbase (scalar) + voff (a lane's offset).
+// those covers it waits for every load in flight, which drains the prefetch). The ring's explicit vmcnt
+// waits and barriers order them instead; the "memory" clobber keeps LDS reads and the barriers on their
+// side of each load. The LDS address (wave-uniform) goes in M0 as an operand the compiler sets, the s_nop
+// the wait state between that write and the load; the global address is sbase (scalar) + voff (a lane's
+// offset).
 __device__ __forceinline__ void to_lds16(const void *sbase, uint32_t voff, void *lds) {
   const uint32_t l = (uint32_t)(uintptr_t)(lds_void *)lds;
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(l) : "memory");
 }
-__device__ __forceinline__ void to_lds4(const void *sbase, uint32_t voff, void *lds) {
+// 2 bytes a lane, each zero-extended to a dword of LDS
+__device__ __forceinline__ void to_lds2(const void *sbase, uint32_t voff, void *lds) {
   const uint32_t l = (uint32_t)(uintptr_t)(lds_void *)lds;
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(l) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_ushort %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(l) : "memory");
 }
 
-// The sources of a lane's loads into LDS: a uniform base (the operand's start plus the step's K
-// offset, in scalar registers) and the lane's byte offset from it (computed once: the loads take the
-// base + offset form, no per-lane address arithmetic a step). Out-of-range rows and columns read the
-// last row/column. The offsets are 32-bit: the launcher takes this form for operands under 4 GiB.
 template <int BM, int BN, bool MX, int WM, int WN, int KG, int RS>
-struct RingSrc {
-  using R = RCfg<BM, BN, MX, WM, WN, KG, RS>;
-  const char *X, *W, *E;
-  uint32_t xo[R::AX], wo[R::AW], eo;
-  uint32_t K;
-  __device__ __forceinline__ RingSrc(const u32x4 *X_, const uint8_t *W_, const uint8_t *E_, uint32_t M, uint32_t N,
-                                     uint32_t K_, uint32_t m0, uint32_t n0, int wave, int lane)
-      : X((const char *)X_), W((const char *)W_), E((const char *)E_), K(K_) {
-#pragma unroll
-    for (int a = 0; a < R::AX; a++) {
-      const int p = (a * R::NW + wave) * 64 + lane, row = p / CH, ch = (p % CH) ^ (row & 15);
-      xo[a] = (min(m0 + row, M - 1) * K + ch * 8) * 2;
-    }
-    const uint32_t rowb = MX ? K / 2 : K;  // weight bytes a column
-#pragma unroll
-    for (int a = 0; a < R::AW; a++) {
-      const int p = (a * R::NW + wave) * 64 + lane, col = p / R::WCH;
-      const int c = (p % R::WCH) ^ ((col / R::CPB) & (R::WCH - 1));
-      wo[a] = min(n0 + col, N - 1) * rowb + c * 16;
-    }
-    eo = MX ? min(n0 + (uint32_t)(wave * 64 + lane), N - 1) * (K / 32) : 0u;  // slots past BN: padding
-  }
-  // The loads of the step at K offset k0 (clamped to the last step: a step past the end rereads it).
-  __device__ __forceinline__ void load(u32x4 *xb, u32x4 *wb, uint32_t *eb, uint32_t k0, int wave) const {
-    k0 = min(k0, K - KS);
-#pragma unroll
-    for (int a = 0; a < R::AX; a++) to_lds16(X + k0 * 2, xo[a], xb + (a * R::NW + wave) * 64);
-#pragma unroll
-    for (int a = 0; a < R::AW; a++) to_lds16(W + (MX ? k0 / 2 : k0), wo[a], wb + (a * R::NW + wave) * 64);
-    if constexpr (MX) to_lds4(E + k0 / 32, eo, eb + wave * 64);
-  }
+struct PairCfg {
+  static constexpr int NW = WM * WN, NT = 64 * NW * KG;  // waves a group; threads
+  static constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
+  static constexpr int WCH = MX ? 2 : 4;                   // 16-byte weight chunks a column a step
+  static constexpr int XI = BM * 8 / 64, WI = BN * WCH / 64, EI = MX ? (BN + 63) / 64 : 0;  // load instructions a step
+  static constexpr int XB = BM * 8, WB = BN * WCH, EB = EI * 16;  // 16-byte slots a stage
+  static constexpr int AX = (XI + NW - 1) / NW, AW = (WI + NW - 1) / NW, AE = (EI + NW - 1) / NW;
+  static constexpr int LMIN = XI / NW + WI / NW + EI / NW;  // the fewest loads a wave issues a step
+  static constexpr int SLOTS = XB + WB + EB;               // a stage
+  static constexpr int STRIP = 16 * (TN * 16 + 4);         // floats of a wave's store strip
+  static constexpr int SUMS = KG > 1 ? KG * BM * BN : 0;   // floats of the groups' tiles
+  static_assert(TM * WM * 16 == BM && TN * WN * 16 == BN && BM % 8 == 0 && BN * WCH % 64 == 0, "tile shape");
+  static constexpr int ENDS = ((SUMS > NW * KG * STRIP ? SUMS : NW * KG * STRIP) + 3) / 4;  // 16-byte slots after the loop
+  static constexpr int LDS = KG * RS * SLOTS > ENDS ? KG * RS * SLOTS : ENDS;
+  static_assert(LMIN * (RS - 2) + 3 * (RS - 2) <= 63, "loads in flight past the wait counter");
 };
 
+// Workgroup id -> tile. Ids x, x+8, x+16, ... share an XCD: each XCD takes a contiguous run of the order
+// below, in which the tiles that run at the same time form a block of kGroupN weight panels by some M tiles,
+// so that each step's X rows and weights are fetched into the XCD's L2 once for all of them. False: no
+// tile (the grid is rounded up to 8).
+constexpr uint32_t kGroupN = 8;
+__host__ __device__ __forceinline__ uint32_t pair_grid(uint32_t tiles) { return (tiles + 7) / 8 * 8; }
+__device__ __forceinline__ bool pair_tile(uint32_t id, uint32_t mt, uint32_t nt, uint32_t &tm, uint32_t &tn) {
+  const uint32_t total = mt * nt, per = (total + 7) / 8;
+  const uint32_t lin = (id % 8) * per + id / 8;
+  if (lin >= total) return false;
+  const uint32_t gr = lin / (kGroupN * mt), r = lin - gr * kGroupN * mt;
+  const uint32_t gn = min(kGroupN, nt - gr * kGroupN);  // panels of the last group
+  tm = r / gn;
+  tn = gr * kGroupN + r % gn;
+  return true;
+}
+
 template <int BM, int BN, bool MX, int WM, int WN, int KG, int RS>
-__device__ __forceinline__ void gemm_ring_wg(uint32_t bx, const u32x4 *__restrict__ X, const uint8_t *__restrict__ W,
+__device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restrict__ X, const uint8_t *__restrict__ W,
                                              const uint8_t *__restrict__ E, const uint16_t *__restrict__ S,
                                              void *__restrict__ Y, uint32_t M, uint32_t N, uint32_t K, int mode,
                                              bool equads) {
-  using C = Cfg<BM, BN, MX, WM, WN, KG>;
-  using R = RCfg<BM, BN, MX, WM, WN, KG, RS>;
-  constexpr int TM = C::TM, TN = C::TN, NT = C::NT, KKG = C::KKG, LS = R::LS;
-  static_assert(RS >= 2 && RS <= 6, "ring depth");
-  // one LDS variable a stage: X, then the weights, then the MXFP4 scales
-  constexpr int XB = BM * CH, WB = R::WSLOTS, EB = MX ? R::NW * 16 : 0;  // 16-byte slots
-  u32x4 *sr[RS], *xr[RS], *wr[RS];
-  uint32_t *er[RS];
-  RingBufs<u32x4, XB + WB + EB, 0, RS>::fill(sr);
-#pragma unroll
-  for (int s = 0; s < RS; s++) {
-    xr[s] = sr[s];
-    wr[s] = sr[s] + XB;
-    er[s] = (uint32_t *)(sr[s] + XB + WB);
-  }
-  __shared__ int hs[MX ? BN : 1], ls[MX ? BN : 1];  // the row shift scan (MXFP4)
-  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int g = wave / (WM * WN), wl = wave % (WM * WN);  // k group, wave in the group
-  const int wm = wl / WN, wn = wl % WN;
+  using C = PairCfg<BM, BN, MX, WM, WN, KG, RS>;
+  constexpr int TM = C::TM, TN = C::TN, NT = C::NT, NW = C::NW, SLOTS = C::SLOTS;
+  __shared__ __attribute__((aligned(16))) u32x4 rings[C::LDS];
+  __shared__ uint32_t flags[NW * KG];
+  const int t = threadIdx.x, lane = t & 63, wg = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int g = wg / NW, wave = wg % NW;  // k group, wave in the group
+  u32x4 *ring = rings + g * RS * SLOTS;
+  const int wm = wave / WN, wn = wave % WN;
   const int r16 = lane & 15, q = lane >> 4;
   uint32_t tm, tn;
-  tile_of(bx, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn);
+  if (!pair_tile(bx, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn)) return;
   const uint32_t m0 = tm * BM, n0 = tn * BN;
   const uint32_t nw = n0 + wn * (BN / WN);  // the wave's first column
-  const uint32_t steps = K / KS;
-  const RingSrc<BM, BN, MX, WM, WN, KG, RS> src(X, W, E, M, N, K, m0, n0, wave, lane);
+  // the group's steps of 64 are h0 .. h1-1; all groups run n_steps of them together (a step past a group's
+  // segment loads in-range data that nothing reads)
+  const uint32_t steps = K / 64, S128 = (steps + 1) / 2;
+  const uint32_t h0 = KG == 1 ? 0 : 2 * seg_first(S128, KG, g);
+  const uint32_t h1 = KG == 1 ? steps : min(2 * seg_first(S128, KG, g + 1), steps);
+  const uint32_t n_steps = KG == 1 ? steps : 2 * ((S128 + KG - 1) / KG);
+
+  // the lane's byte offsets of its loads from the operand's start plus the step's K offset (32-bit: the
+  // launcher takes this form for operands under 4 GiB); rows and columns past the end read the last
+  uint32_t xo[C::AX], wo[C::AW], eo[C::AE > 0 ? C::AE : 1];
 #pragma unroll
-  for (int s = 0; s < RS - 1; s++) src.load(xr[s], wr[s], er[s], s * KS, wave);
-  int s0[TN];
-#pragma unroll
-  for (int j = 0; j < TN; j++) s0[j] = 0;
-  if constexpr (MX) {
-    if (t < BN) {
-      hs[t] = 0;
-      ls[t] = 255;
-    }
-    wait_lds();
-    ring_barrier();
-    scan_shifts<BN, NT>(E, n0, N, K / 32, equads, t, hs, ls);
-    wait_lds();
-    ring_barrier();
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-      const uint32_t r = min(nw + j * 16 + r16, N - 1) - n0;
-      s0[j] = shift_of(hs[r], ls[r]);
-    }
+  for (int a = 0; a < C::AX; a++) {
+    const int p = (a * NW + wave) * 64 + lane, row = p / 8, ch = (p % 8) ^ ((row >> 1) & 7);
+    xo[a] = (min(m0 + row, M - 1) * K + ch * 8) * 2;
   }
+#pragma unroll
+  for (int a = 0; a < C::AW; a++) {
+    const int p = (a * NW + wave) * 64 + lane, col = p / C::WCH;
+    const int c = (p % C::WCH) ^ (MX ? (col >> 3) & 1 : (col >> 2) & 3);
+    wo[a] = min(n0 + col, N - 1) * (MX ? K / 2 : K) + c * 16;
+  }
+#pragma unroll
+  for (int a = 0; a < C::AE; a++) eo[a] = min(n0 + (uint32_t)((a * NW + wave) * 64 + lane), N - 1) * (K / 32);
+  auto load = [&](uint32_t j, int s) __attribute__((always_inline)) {
+    const uint32_t k0 = min(h0 + j, steps - 1) * 64;
+    u32x4 *xb = ring + s * SLOTS, *wb = xb + C::XB;
+    uint32_t *eb = (uint32_t *)(wb + C::WB);
+#pragma unroll
+    for (int a = 0; a < C::AX; a++)
+      if (C::XI % NW == 0 || a * NW + wave < C::XI)
+        to_lds16((const char *)X + k0 * 2, xo[a], xb + (a * NW + wave) * 64);
+#pragma unroll
+    for (int a = 0; a < C::AW; a++)
+      if (C::WI % NW == 0 || a * NW + wave < C::WI)
+        to_lds16((const char *)W + (MX ? k0 / 2 : k0), wo[a], wb + (a * NW + wave) * 64);
+#pragma unroll
+    for (int a = 0; a < C::AE; a++)
+      if (C::EI % NW == 0 || a * NW + wave < C::EI)
+        to_lds2((const char *)E + k0 / 32, eo[a], eb + (a * NW + wave) * 64);
+  };
+  // this wave's loads of all steps but the last RS - 2 issued done
+  const int extra = (wave < C::XI % NW) + (wave < C::WI % NW) + (wave < C::EI % NW);
+  auto wait_step = [&]() __attribute__((always_inline)) {
+    if (extra == 0) wait_loads<C::LMIN * (RS - 2)>();
+    else if (extra == 1) wait_loads<(C::LMIN + 1) * (RS - 2)>();
+    else if (extra == 2) wait_loads<(C::LMIN + 2) * (RS - 2)>();
+    else wait_loads<(C::LMIN + 3) * (RS - 2)>();
+  };
 
   floatx4 acc[TM][TN];
+  int s0[TN];
+  uint32_t lo = 104, hi = 140;
 #pragma unroll
-  for (int i = 0; i < TM; i++)
+  for (int j = 0; j < TN; j++) s0[j] = 0;
+  // the lane's operands in a stage: X rows of 16 apart, weight columns of 16 apart
+  const uint32_t xa = (wm * (BM / WM) + r16) * 128, wa = (wn * (BN / WN) + r16) * (C::WCH * 16);
+  const uint32_t xsw = (r16 >> 1) & 7;
+  const uint32_t wsl = MX ? (((q >> 1) ^ ((r16 >> 3) & 1)) * 16 + (q & 1) * 8) : (q ^ ((r16 >> 2) & 3)) * 16;
+  const uint32_t ea = (wn * (BN / WN) + r16) * 4 + (q >> 1);
+  auto main_loop = [&](auto shifted) __attribute__((always_inline)) {
+    constexpr bool SHIFT = decltype(shifted)::value;
 #pragma unroll
-    for (int j = 0; j < TN; j++) acc[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
-
-  // Software-pipelined steps: the operands of step j+1 are read from LDS (into the other register set)
-  // before the MFMAs of step j, so that the LDS reads of one step run under the MFMAs of the other
-  // (every operand of a step read at once: read one at a time before its MFMA, each read's latency
-  // showed). Step j: wait for this wave's LDS reads of step j (in registers: buffer j % RS is free)
-  // and its loads of step j+1, a barrier (every wave's loads of step j+1 have landed, every wave is
-  // done with buffer j % RS), the reads of step j+1, the loads of step j+RS into buffer j % RS, then
-  // the MFMAs of step j, each kk's weights converted next to the MFMAs that take them.
-  struct Ops {
-    u32x4 ax[KKG][TM];
-    u32x4 wv[TN][C::BL];  // int8: the wave's codes of the step
-    u32x2 wd[TN];         // MXFP4: the k group's dwords of block q (KG 2) or the first two (KG 1)
-    u32x2 wd2[TN];        // MXFP4 KG 1: the last two
-    uint32_t eb[TN];      // MXFP4: the block scale bytes of the step (4 a dword)
-  };
-  auto read_ops = [&](Ops &o, int b) __attribute__((always_inline)) {
-    const u32x4 *xb = xr[b], *wb = wr[b];
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-    for (int jn = 0; jn < TN; jn++) {
-      const int col = wn * (BN / WN) + jn * 16 + r16;
-      if constexpr (MX) {
-        const int slot = col * R::WCH + (q ^ ((col / R::CPB) & (R::WCH - 1)));
-        if constexpr (KG == 1) {
-          const u32x4 v = wb[slot];
-          o.wd[jn] = (u32x2){v[0], v[1]};
-          o.wd2[jn] = (u32x2){v[2], v[3]};
-        } else {
-          o.wd[jn] = *((const u32x2 *)&wb[slot] + g);
-        }
-        o.eb[jn] = er[b][col];
-      } else {
+      for (int j = 0; j < TN; j++) acc[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int h = 0; h < C::BL; h++) {
-          const int c = (KG == 1 ? h : g) * 4 + q;
-          o.wv[jn][h] = wb[col * R::WCH + (c ^ ((col / R::CPB) & (R::WCH - 1)))];
-        }
-      }
-    }
+    for (int s = 0; s < RS - 1; s++) load(s, s);
+    for (uint32_t j0 = 0; j0 < n_steps; j0 += RS) {
 #pragma unroll
-    for (int kk = 0; kk < KKG; kk++)
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        const int row = wm * (BM / WM) + i * 16 + r16;
-        const int ch = KG == 1 ? xchunk<MX>(q, kk) : xchunk<MX>(q, g * KKG + kk);
-        o.ax[kk][i] = xb[row * CH + (ch ^ (row & 15))];
-      }
-  };
-  auto mfma_ops = [&](const Ops &o) __attribute__((always_inline)) {
-    float sc[TN];
-    if constexpr (MX) {
-#pragma unroll
-      for (int jn = 0; jn < TN; jn++) sc[jn] = shifted_scale((o.eb[jn] >> (8 * q)) & 255u, s0[jn]);
-    }
-    auto bops = [&](half8 (&bf)[TN], int kk) __attribute__((always_inline)) {
-#pragma unroll
-      for (int jn = 0; jn < TN; jn++) {
-        if constexpr (MX) {
-          const uint32_t w = KG == 1 ? (kk < 2 ? o.wd[jn][kk] : o.wd2[jn][kk - 2]) : o.wd[jn][kk];
-          bf[jn] = fp4x8_to_half8(w, sc[jn]);
-        } else {
-          const u32x4 v = o.wv[jn][kk >> 1];
-          bf[jn] = i8x8_to_half8(v[(kk & 1) * 2], v[(kk & 1) * 2 + 1]);
-        }
-      }
-    };
-    half8 bf[2][TN];
-    bops(bf[0], 0);
-#pragma unroll
-    for (int kk = 0; kk < KKG; kk++) {
-      if (kk + 1 < KKG) bops(bf[(kk + 1) & 1], kk + 1);
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int jn = 0; jn < TN; jn++)
-          acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, o.ax[kk][i]), bf[kk & 1][jn],
-                                                              acc[i][jn], 0, 0, 0);
-    }
-  };
-  Ops P[2];
-  wait_loads<(RS - 2) * LS>();  // step 0 (this wave's loads)
-  ring_barrier();
-  issue_order();
-  src.load(xr[RS - 1], wr[RS - 1], er[RS - 1], (RS - 1) * KS, wave);
-  issue_order();
-  read_ops(P[0], 0);
-  for (uint32_t j0 = 0; j0 < steps; j0 += 2 * RS) {
-#pragma unroll
-    for (int s = 0; s < 2 * RS; s++) {
-      const uint32_t j = j0 + s;
-      if (j >= steps) break;
-      wait_lds();  // this wave's reads of step j (on both paths: the MFMAs below then wait for nothing)
-      if (j + 1 < steps) {
-        wait_loads<(RS - 2) * LS>();
+      for (int s = 0; s < RS; s++) {
+        const uint32_t j = j0 + s;
+        if (j >= n_steps) break;
+        // every wave's loads of step j landed, every wave done with step j-1's stage, which step j+RS-1 takes
+        wait_step();
+        wait_lds();
         ring_barrier();
         issue_order();
-        read_ops(P[(s + 1) & 1], (s + 1) % RS);
+        load(j + RS - 1, (s + RS - 1) % RS);
         issue_order();
-        src.load(xr[s % RS], wr[s % RS], er[s % RS], (j + RS) * KS, wave);
-        issue_order();
+        if (KG > 1 && h0 + j >= h1) continue;
+        const char *xb = (const char *)(ring + s * SLOTS), *wb = xb + C::XB * 16, *eb = wb + C::WB * 16;
+        u32x2 wc[MX ? TN : 1];
+        u32x4 wv[MX ? 1 : TN];
+        float sc[TN];
+#pragma unroll
+        for (int jn = 0; jn < TN; jn++) {
+          if constexpr (MX) {
+            wc[jn] = *(const u32x2 *)(wb + wa + jn * 16 * 32 + wsl);
+            const uint32_t e = *(const uint8_t *)(eb + ea + jn * 64);
+            sc[jn] = SHIFT ? shifted_scale(e, s0[jn]) : __uint_as_float(e << 23);
+            if constexpr (!SHIFT) {
+              lo = min(lo, e);
+              hi = max(hi, e);
+            }
+          } else {
+            wv[jn] = *(const u32x4 *)(wb + wa + jn * 16 * 64 + wsl);
+          }
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+          half8 af[TM], bf[TN];
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+            af[i] = __builtin_bit_cast(half8, *(const u32x4 *)(xb + xa + i * 16 * 128 + ((2 * q + kk) ^ xsw) * 16));
+#pragma unroll
+          for (int jn = 0; jn < TN; jn++) {
+            if constexpr (MX) bf[jn] = fp4x8_to_half8(wc[jn][kk], sc[jn]);
+            else bf[jn] = i8x8_to_half8(wv[jn][kk * 2], wv[jn][kk * 2 + 1]);
+          }
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int jn = 0; jn < TN; jn++)
+              acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[jn], acc[i][jn], 0, 0, 0);
+        }
       }
-      mfma_ops(P[s & 1]);
+    }
+    wait_loads<0>();  // no load into LDS may land in a stage put to another use
+  };
+  main_loop(std::false_type{});
+  bool shift = false;
+  if constexpr (MX) {
+    // a scale whose exponent leaves [-23, 13] (or a zero or infinite one): the tile again, its rows shifted
+    if (__ballot(lo < 104 || hi > 140)) shift = true;
+    if (lane == 0) flags[wg] = shift;
+  }
+  wait_lds();
+  ring_barrier();  // every wave is done with the stages
+  if constexpr (MX) {
+    shift = false;
+#pragma unroll
+    for (int w = 0; w < NW * KG; w++) shift |= flags[w] != 0;
+    shift = __builtin_amdgcn_readfirstlane(shift);
+    if (shift) {
+      int *hs = (int *)rings, *ls = hs + BN;
+      for (int i = t; i < BN; i += NT) {
+        hs[i] = 0;
+        ls[i] = 255;
+      }
+      __syncthreads();
+      scan_shifts<BN, NT>(E, n0, N, K / 32, equads, t, hs, ls);
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const uint32_t r = min(nw + j * 16 + r16, N - 1) - n0;
+        s0[j] = shift_of(hs[r], ls[r]);
+      }
+      __syncthreads();
+      main_loop(std::true_type{});
+      wait_lds();
+      ring_barrier();
     }
   }
-  wait_loads<0>();  // no load into LDS may land after the workgroup ends
-  if constexpr (KG == 2) {
-    // group 1's accumulators to group 0 through the X buffers, summed in group 0, which writes the
-    // tile (BM x BN fp32: 2 buffers hold BM x 128)
-    static_assert(BM * BN * 4 <= 2 * BM * CH * 16, "the k groups' sum goes through two X buffers");
-    constexpr int HALF = BM * CH;  // float4 slots a buffer
+  if constexpr (KG > 1) {
+    // the groups' tiles through LDS: the wave of group g sums rows i = g, g + KG, ... (16 each) of its block,
+    // in the order of the segments, and stores them
+    floatx4 *sums = (floatx4 *)rings;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      if (i % KG == g) continue;
+#pragma unroll
+      for (int j = 0; j < TN; j++) sums[(((g * NW + wave) * TM + i) * TN + j) * 64 + lane] = acc[i][j];
+    }
     wait_lds();
     ring_barrier();
-    if (g == 1) {
 #pragma unroll
-      for (int i = 0; i < TM; i++)
+    for (int i = 0; i < TM; i++) {
+      if (i % KG != g) continue;
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-          const int r = ((wl * TM + i) * TN + j) * 64;  // wave-uniform
-          floatx4 *d = r < HALF ? (floatx4 *)xr[0] + r : (floatx4 *)xr[1] + (r - HALF);
-          d[lane] = acc[i][j];
+      for (int j = 0; j < TN; j++) {
+        floatx4 v;
+#pragma unroll
+        for (int k = 0; k < KG; k++) {
+          const floatx4 p = k == g ? acc[i][j] : sums[(((k * NW + wave) * TM + i) * TN + j) * 64 + lane];
+          v = k == 0 ? p : v + p;
         }
-    }
-    wait_lds();
-    ring_barrier();
-    if (g == 0) {
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-          const int r = ((wl * TM + i) * TN + j) * 64;
-          const floatx4 *d = r < HALF ? (const floatx4 *)xr[0] + r : (const floatx4 *)xr[1] + (r - HALF);
-          acc[i][j] += d[lane];
-        }
-    }
-    wait_lds();
-    ring_barrier();  // group 0 is done with the sums' buffers, which its stores reuse
-    if (g == 1) return;
-  }
-  // staged stores where the waves' blocks fit the X buffers (a wave's block in region wl, PER regions
-  // a buffer), else straight from the accumulators
-  using G = StageRows<TM, TN, TN * 16 + 4>;
-  constexpr int PER = BM * CH * 4 / G::FLOATS;
-  if constexpr (PER >= 1 && (WM * WN + PER - 1) / PER <= RS) {
-    if (staged(Y, N, mode)) {
-      if constexpr (KG == 1) {
-        wait_lds();
-        ring_barrier();  // every wave is done with the ring's buffers
+        acc[i][j] = v;
       }
-      store_tile_staged<BM, WM, TM, TN, MX, TN * 16 + 4>(acc, s0, S, Y, M, N, m0, nw, wm, lane, mode,
-                                                         (float *)xr[wl / PER] + (wl % PER) * G::FLOATS);
-      return;
     }
+    wait_lds();
+    ring_barrier();  // the sums are read: the store strips take their place
   }
-  store_tile<BM, WM, TM, TN, MX>(acc, s0, S, Y, M, N, m0, nw, wm, r16, q, mode);
+  if (staged(Y, N, mode))
+    store_strips<TM, TN, MX, KG>(acc, s0, shift, S, Y, M, N, m0 + wm * (BM / WM), nw, lane, mode,
+                                 (float *)rings + wg * C::STRIP, g);
+  else
+    store_tile<BM, WM, TM, TN, MX, KG>(acc, s0, S, Y, M, N, m0, nw, wm, r16, q, mode, g);
 }
 
 }  // namespace hwk_gemm

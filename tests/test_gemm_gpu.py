@@ -134,3 +134,64 @@ def test_gemm_swiglu_rejects_ragged_n(dev):
     w, e = synth.mxfp4_normal(24, 64, "k3swr.w", std=0.02)
     with pytest.raises(Exception, match="SwiGLU"):
         ops.mxfp4_gemm(x, w, e, "swiglu")
+
+
+# One case a tile of the paired form (hwk_gemm's HWK_PAIR_MX / HWK_PAIR_I8, in the tables' order, as pick_pair
+# chooses them), each with rows and columns left over: first with one step of 64 values (fewer than its k
+# groups and ring stages), then with several (a number that its k groups do not divide).
+PAIR_MX = [(898, 6152, 64), (898, 4100, 64), (450, 4100, 64), (289, 4100, 64), (198, 4100, 64), (65, 6152, 64),
+           (37, 4100, 64), (23, 4100, 64), (9, 130, 64)]
+PAIR_I8 = [(898, 4100, 64), (387, 6152, 64), (450, 4100, 64), (198, 4100, 64), (65, 6152, 64), (37, 4100, 64),
+           (23, 4100, 64), (9, 130, 64)]
+PAIR_K = 832
+
+
+@pytest.mark.parametrize("k", [64, 192, PAIR_K])
+@pytest.mark.parametrize("mx,m,n", [(True, m, n) for m, n, _ in PAIR_MX] + [(False, m, n) for m, n, _ in PAIR_I8])
+def test_gemm_paired_tiles(dev, orc, mx, m, n, k):
+    """The paired form's tiles against the oracle in fp32, and their fp16 and added results against their fp32
+    ones bit for bit."""
+    print(f"gemm tiles mx={mx} {m}x{n}x{k}", flush=True)
+    name = f"k3pair.{mx}.{m}.{n}.{k}"
+    x = synth.normal(m * k, name + ".x").view(m, k)
+    if mx:
+        w, e = synth.mxfp4_normal(n, k, name + ".w", std=0.02)
+        wd = orc.mxfp4_dequantize(w.cpu().numpy(), e.cpu().numpy())
+        run = lambda mode, y=None: ops.mxfp4_gemm(x, w, e, mode, y=y)  # noqa: E731
+    else:
+        q = synth.uniform_int(n * k, -127, 255, name + ".q", dtype=torch.int8).view(n, k)
+        s = synth.uniform_real(n, 0.002, 0.02, name + ".s")
+        wd = orc.i8_dequant(q.cpu().numpy(), s.cpu().numpy().view(np.uint16))
+        run = lambda mode, y=None: ops.i8_gemm(x, q, s, mode, y=y)  # noqa: E731
+    want = orc.sgemm(x.cpu().numpy().astype(np.float32), wd, transb=True)
+    y32 = run("f32").cpu().numpy()
+    check_close(y32, want)
+    assert np.array_equal(run("f16").cpu().numpy().view(np.uint16), orc.f32_to_f16(y32))
+    y0 = synth.normal(m * n, name + ".y0", dtype=torch.float32).view(m, n)
+    b0 = y0.cpu().numpy()
+    run("add", y0)
+    assert np.array_equal(y0.cpu().numpy(), (b0 + y32).astype(np.float32))
+
+
+@pytest.mark.parametrize("m,n,k", [(898, 6144, 64), (450, 4096, 192), (65, 6144, 192), (9, 128, PAIR_K)])
+def test_mxfp4_gemm_shifted_tiles(dev, orc, m, n, k):
+    """Rows whose exponents leave [-23, 13] in single tiles of a wide product (one k group and several): those
+    tiles run again with their rows shifted, the others do not, and every column meets the oracle at its
+    own size; the SwiGLU output equals that of the fp32 one."""
+    rng = np.random.default_rng(m + n)
+    x = synth.normal(m * k, f"k3shift.{m}.x").view(m, k)
+    w = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    e = rng.integers(127 - 9, 127 - 6, (n, k // 32))
+    e[5] = 127 + 15 + np.arange(k // 32) % 4
+    e[n // 2 + 3] = 127 - 30 - np.arange(k // 32) % 3
+    e[n - 1, ::2] = 0
+    e = e.astype(np.uint8)
+    want = orc.sgemm(x.cpu().numpy().astype(np.float32), orc.mxfp4_dequantize(w, e), transb=True)
+    wt, et = torch.from_numpy(w).cuda(), torch.from_numpy(e).cuda()
+    y = ops.mxfp4_gemm(x, wt, et, "f32")
+    got = y.cpu().numpy().astype(np.float64)
+    col = np.sqrt(np.mean(want.astype(np.float64) ** 2, 0))
+    assert np.all(np.max(np.abs(got - want), 0) <= TOL * col)
+    flat = y.view(-1)
+    want16 = ops.silu_mul(flat, flat[1:], "f16", stride=2, n=m * n // 2).view(m, n // 2)
+    assert torch.equal(ops.mxfp4_gemm(x, wt, et, "swiglu").view(torch.int16), want16.view(torch.int16))
