@@ -53,6 +53,9 @@ char *attn_step(hipStream_t st, const float *qkv, const float *qn, const float *
                 void *kc, void *vc, void *workspace, size_t workspace_bytes, const hwk_attn_params *p,
                 const int32_t *pos, bool keep);
 
+// The most workspace that hwk_attn_prefill_ws asks for in a cache of max_ctx positions.
+size_t attn_prefill_most_bytes(uint32_t max_ctx);
+
 }  // namespace hwk
 
 // A double's DPP move (both halves moved alike; lanes the row mask leaves out get 0.0).

@@ -436,7 +436,7 @@ char *prefill_piece(hwk_qwen3 *m, hipStream_t st, uint32_t T, uint32_t start, bo
     hipLaunchKernelGGL(k_qk_rope, dim3((slots + 3) / 4, T), dim3(256), 0, st, m->qkv, ly.q_norm, ly.k_norm, m->cos_t,
                        m->sin_t, m->pos, 0u, m->q16, ly.kc, ly.vc, c.heads, c.kv_heads, c.max_ctx, m->eps);
     HWK_Q(hwk::launched("qwen3 qk_rope"));
-    HWK_Q(hwk_attn_prefill(st, m->q16, ly.kc, ly.vc, m->att16, T, start, &pp));
+    HWK_Q(hwk_attn_prefill_ws(st, m->q16, ly.kc, ly.vc, m->att16, m->ws, m->ws_bytes, T, start, &pp));
     HWK_Q(hwk_mxfp4_gemm(st, m->att16, ly.o.w, ly.o.e, m->h, T, c.hidden, m->att_n, HWK_OUT_ADD_F32));
     HWK_Q(hwk::rmsnorm_f16(st, m->h, ly.post_norm, m->eps, m->x16, T, c.hidden));
     HWK_Q(hwk_mxfp4_gemm(st, m->x16, ly.gu.w, ly.gu.e, m->a16, T, 2 * c.inter, c.hidden, HWK_OUT_SWIGLU_F16));
@@ -485,7 +485,7 @@ char *verify_piece(hwk_qwen3 *m, hipStream_t st, uint32_t T, uint32_t start) {
     hipLaunchKernelGGL(k_qk_rope, dim3((slots + 3) / 4, T), dim3(256), 0, st, m->qkv, ly.q_norm, ly.k_norm, m->cos_t,
                        m->sin_t, m->pos, 0u, m->q16, ly.kc, ly.vc, c.heads, c.kv_heads, c.max_ctx, m->eps);
     HWK_Q(hwk::launched("qwen3 verify qk_rope"));
-    HWK_Q(hwk_attn_prefill(st, m->q16, ly.kc, ly.vc, m->att16, T, start, &pp));
+    HWK_Q(hwk_attn_prefill_ws(st, m->q16, ly.kc, ly.vc, m->att16, m->ws, m->ws_bytes, T, start, &pp));
     HWK_Q(rows_linear(st, m->att16, ly.o, m->h, T, HWK_OUT_ADD_F32));
     HWK_Q(hwk::rmsnorm_f16(st, m->h, ly.post_norm, m->eps, m->x16, T, c.hidden));
     HWK_Q(rows_linear(st, m->x16, ly.gu, m->gu, T, HWK_OUT_F32));
@@ -536,7 +536,8 @@ HWK_API char *hwk_qwen3_new(const hwk_qwen3_config *cfg, hwk_qwen3 **out) {
   ap.out_mode = HWK_OUT_F16;
   ap.split = 0;
   hwk::attn_step_layout(&ap, &m->step_chunk, &m->step_nchunk);
-  m->ws_bytes = hwk::attn_step_workspace_bytes(&ap);
+  // the states of split attention: a step's chunks, or a prompt's or a verify's (never both at once)
+  m->ws_bytes = std::max(hwk::attn_step_workspace_bytes(&ap), hwk::attn_prefill_most_bytes(c.max_ctx));
   {
     const uint64_t row = (uint64_t)c.layers * c.kv_heads * c.head_dim * 2 * sizeof(uint16_t);
     m->keep_rows = (uint32_t)std::min<uint64_t>(kKeepCacheBytes / row, c.max_ctx);

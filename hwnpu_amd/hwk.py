@@ -136,6 +136,8 @@ SIGNATURES = {
     "hwk_kv_quantize_i8": (ERR, [P, P, P, P, U32, U32]),
     "hwk_attn_merge": (ERR, [P, P, P, P, P, U32, U32, U32, C.c_int]),
     "hwk_attn_prefill": (ERR, [P, P, P, P, P, U32, U32, C.POINTER(AttnParams)]),
+    "hwk_attn_prefill_workspace_bytes": (SZ, [U32, U32, C.POINTER(AttnParams)]),
+    "hwk_attn_prefill_ws": (ERR, [P, P, P, P, P, P, SZ, U32, U32, C.POINTER(AttnParams)]),
     "hwk_qwen3_new": (ERR, [C.POINTER(Qwen3Config), C.POINTER(P)]),
     "hwk_qwen3_free": (None, [P]),
     "hwk_qwen3_synth": (ERR, [P, P, U64, U32]),

@@ -256,7 +256,11 @@ def attn_prefill(q, k, v, start, out_mode="f32", scale=None, out=None):
         out = torch.empty((tokens, heads, d), dtype=dt, device=q.device)
     else:
         _need(out, "out", dt, (tokens, heads, d))
-    hwk.load().hwk_attn_prefill(_stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), tokens, start, p)
+    lib = hwk.load()
+    n = lib.hwk_attn_prefill_workspace_bytes(tokens, start, p)
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
+    lib.hwk_attn_prefill_ws(_stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _ptr(ws), n, tokens,
+                            start, p)
     return out
 
 

@@ -312,6 +312,14 @@ HWK_API char *hwk_kv_quantize_i8(void *stream, const void *x, void *q, void *sca
  * prompt through it, internal/llm/decode/decode.go:1391-1483). */
 HWK_API char *hwk_attn_prefill(void *stream, const void *q, const void *k, const void *v, void *out,
                                uint32_t tokens, uint32_t start, const hwk_attn_params *p);
+/* hwk_attn_prefill with device memory for the partial outputs of keys split over workgroups, which a few
+ * rows behind a long cache need to fill the chip: hwk_attn_prefill_workspace_bytes of it (0: none, it may be
+ * NULL), 16-byte aligned, no initial contents. Calls that overlap on one workspace race. The results differ
+ * from hwk_attn_prefill's by the order of fp32 sums. */
+HWK_API size_t hwk_attn_prefill_workspace_bytes(uint32_t tokens, uint32_t start, const hwk_attn_params *p);
+HWK_API char *hwk_attn_prefill_ws(void *stream, const void *q, const void *k, const void *v, void *out,
+                                  void *workspace, size_t workspace_bytes, uint32_t tokens, uint32_t start,
+                                  const hwk_attn_params *p);
 /* Merge chunk outputs as the reference's Merge does (paged.go:227-310): o (chunks, rows, dim)
  * fp32, each chunk normalized over its own keys, m and l (chunks, rows) fp32 (a chunk whose l is
  * not positive is skipped); out (rows, dim) per out_mode, zero for a row no chunk saw. */

@@ -211,3 +211,76 @@ def test_attn_prefill_causal(dev, orc, heads, kvh, T, start, cap):
     # the last row equals decode attention at that position
     dec = ops.attn_decode(q[T - 1].contiguous(), k, v, start + T).cpu().numpy()
     check_close(got[T - 1], dec)
+
+
+# split over workgroups with a workspace (hwk_attn_prefill_ws): one row, a few, blocks whose last rows are
+# missing, chunks that end inside the causal edge, the most chunks (64); each also without the workspace
+@pytest.mark.parametrize("heads,kvh,T,start,cap", [
+    (16, 8, 1, 511, 512), (16, 8, 5, 1024, 1280), (8, 8, 8, 3000, 3072), (32, 8, 33, 1500, 1536), (16, 8, 64, 2000, 2064),
+    (32, 8, 130, 4000, 4200), (4, 1, 3, 9000, 9003), (2, 2, 65, 700, 800)])
+def test_attn_prefill_split(dev, orc, heads, kvh, T, start, cap):
+    print(f"attn prefill split heads={heads} kv={kvh} T={T} start={start} cap={cap}", flush=True)
+    from hwnpu_amd import hwk
+
+    name = f"c3s.{heads}.{T}.{start}"
+    q = synth.normal(T * heads * 128, name + ".q").view(T, heads, 128)
+    k = synth.normal(kvh * cap * 128, name + ".k").view(kvh, cap, 128)
+    v = synth.normal(kvh * cap * 128, name + ".v").view(kvh, cap, 128)
+    k[:, start + T:], v[:, start + T:] = float("nan"), float("nan")  # past the keys: never part of a result
+    scale = 1 / math.sqrt(128)
+    p = ops.attn_params(heads, kvh, start + T, cap)
+    assert hwk.load().hwk_attn_prefill_workspace_bytes(T, start, p) > 0
+    want = oracle_prefill(orc, q.cpu().numpy().astype(np.float32), k.cpu().numpy().astype(np.float32),
+                          v.cpu().numpy().astype(np.float32), start, scale)
+    got = ops.attn_prefill(q, k, v, start, out_mode="f32").cpu().numpy()
+    whole = torch.empty((T, heads, 128), dtype=torch.float32, device="cuda")
+    hwk.load().hwk_attn_prefill(ops._stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(), whole.data_ptr(), T, start, p)
+    whole = whole.cpu().numpy()
+    for t in range(T):
+        check_close(got[t], want[t])
+        check_close(whole[t], want[t])
+    g16 = ops.attn_prefill(q, k, v, start, out_mode="f16").cpu().numpy()
+    assert np.array_equal(g16.view(np.uint16), orc.f32_to_f16(got))
+
+
+def test_attn_prefill_workspace_checked(dev):
+    """A workspace that is missing, short or misaligned is refused; none is needed for a short prompt."""
+    from hwnpu_amd import hwk
+
+    lib = hwk.load()
+    q = synth.normal(5 * 16 * 128, "c3w.q").view(5, 16, 128)
+    k = synth.normal(8 * 2048 * 128, "c3w.k").view(8, 2048, 128)
+    out = torch.empty((5, 16, 128), dtype=torch.float32, device="cuda")
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    ptr = [t.data_ptr() for t in (q, k, k, out)]
+    p = ops.attn_params(16, 8, 2005, 2048)
+    need = lib.hwk_attn_prefill_workspace_bytes(5, 2000, p)
+    assert need > 0
+    for w, n in ((None, need), (ws.data_ptr(), need - 1), (ws.data_ptr() + 4, need)):
+        with pytest.raises(hwk.HwkError, match="workspace"):
+            lib.hwk_attn_prefill_ws(ops._stream(), *ptr, w, n, 5, 2000, p)
+    p = ops.attn_params(16, 8, 5, 2048)
+    assert lib.hwk_attn_prefill_workspace_bytes(5, 0, p) == 0
+    lib.hwk_attn_prefill_ws(ops._stream(), *ptr, None, 0, 5, 0, p)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("scale", [-0.09, 0.0, 3.0])
+@pytest.mark.parametrize("T,start", [(40, 90), (3, 900)])
+def test_attn_prefill_scales(dev, T, start, scale):
+    """Scales of either sign, zero (a plain mean of the visible values) and one large enough that a row's
+    running maximum moves far between tiles, against float64 softmax; bound: P.V sums of at most 940 fp32
+    probabilities (each below 2^-23 off after exp2 of a score whose rounding is |s| 2^-24 log2 e)."""
+    heads, kvh, cap = 4, 2, 1024
+    q = synth.normal(T * heads * 128, f"c3z.{T}.q").view(T, heads, 128)
+    k = synth.normal(kvh * cap * 128, f"c3z.{T}.k").view(kvh, cap, 128)
+    v = synth.normal(kvh * cap * 128, f"c3z.{T}.v").view(kvh, cap, 128)
+    got = ops.attn_prefill(q, k, v, start, out_mode="f32", scale=scale).cpu().double()
+    qd, kd, vd = q.cpu().double(), k.cpu().double(), v.cpu().double()
+    see = torch.arange(start + T)[None] <= start + torch.arange(T)[:, None]
+    sc = float(np.float32(scale))
+    for h in range(heads):
+        s = qd[:, h] @ kd[h // 2, :start + T].T * sc
+        want = torch.softmax(s.masked_fill(~see, -math.inf), -1) @ vd[h // 2, :start + T]
+        lim = 2e-6 + float(s.abs().max()) * 2.0 ** -22
+        assert float((got[:, h] - want).abs().max()) <= lim * float(want.abs().max())
