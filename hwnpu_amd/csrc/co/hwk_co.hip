@@ -145,6 +145,7 @@ __device__ __forceinline__ hwk_moe::MoeArgs moe_args(uint32_t T, uint32_t H, uin
   a.limit = __uint_as_float(limit_bits);
   a.scale = 0.0f;
   a.mode = (int)mode;
+  a.span = 1;
   return a;
 }
 
@@ -262,8 +263,9 @@ __global__ __launch_bounds__(256) void hwk_co_moe_gate_up(const uint4 *__restric
     return;
   }
   const uint32_t gx = (I + 7) / 8;
-  hwk_moe::moe_gate_up_wg<1, 2, false>(blockIdx.x % gx, blockIdx.x / gx, x, nullptr, nullptr, const_cast<int32_t *>(idx),
-                                       nullptr, gw, ge, gb, act, moe_args(T, H, I, E, k, act_kind, alpha_bits, limit_bits, 0));
+  __shared__ __attribute__((aligned(16))) char xs[8 * 4096];  // x_bytes of 8 tokens
+  hwk_moe::moe_gate_up_wg<32, 2, 2, false>(blockIdx.x % gx, blockIdx.x / gx, x, nullptr, nullptr, const_cast<int32_t *>(idx),
+                                       nullptr, gw, ge, gb, act, moe_args(T, H, I, E, k, act_kind, alpha_bits, limit_bits, 0), xs);
 }
 
 // down (E, H, I/32, 16) codes, (E, H, I/32) scales, optional fp32 biases (E, H), of act (T, k, I):
@@ -279,7 +281,7 @@ __global__ __launch_bounds__(512) void hwk_co_moe_down(const float *__restrict__
     if (T <= 8 && t < T && r < H && H <= 8192) out[(size_t)t * H + r] = __builtin_nanf("");
     return;
   }
-  hwk_moe::moe_down_wg<8, 3, 2, false, 8>(blockIdx.x, act, idx, w, dw, de, db, out,
+  hwk_moe::moe_down_wg<8, 3, 1, 8>(blockIdx.x, act, idx, w, dw, de, db, out,
                                           moe_args(T, H, I, E, k, HWK_ACT_SILU, 0, 0, mode));
 }
 

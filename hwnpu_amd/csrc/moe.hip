@@ -21,62 +21,50 @@ __global__ __launch_bounds__(256) void k_moe_route(const float *__restrict__ log
   choose_wave(logits + (size_t)row * E, bias, E, k, score, norm, scale, idx + (size_t)row * k, w + (size_t)row * k);
 }
 
-template <int BPL, int PPW, bool ROUTE>
+template <int LPR, int BPL, int PPW, bool ROUTE>
 __global__ __launch_bounds__(256) void k_moe_gate_up(const uint4 *__restrict__ x, const float *__restrict__ logits,
                                                      const float *__restrict__ rbias, int32_t *__restrict__ idx,
                                                      float *__restrict__ wout, const uint4 *__restrict__ gw,
                                                      const uint8_t *__restrict__ ge, const float *__restrict__ gb,
                                                      float *__restrict__ act, MoeArgs a) {
-  moe_gate_up_wg<BPL, PPW, ROUTE>(blockIdx.x, blockIdx.y, x, logits, rbias, idx, wout, gw, ge, gb, act, a);
+  extern __shared__ __attribute__((aligned(16))) char xs[];
+  moe_gate_up_wg<LPR, BPL, PPW, ROUTE>(blockIdx.x, blockIdx.y, x, logits, rbias, idx, wout, gw, ge, gb, act, a, xs);
 }
 
-template <int LPR, int BPL, int EPW, bool AL, int NW>
+template <int LPR, int BPL, int R, int NW>
 __global__ __launch_bounds__(64 * NW) void k_moe_down(const float *__restrict__ act, const int32_t *__restrict__ idx,
-                                                  const float *__restrict__ w, const uint4 *__restrict__ dw,
-                                                  const uint8_t *__restrict__ de, const float *__restrict__ db,
-                                                  float *__restrict__ out, MoeArgs a) {
-  moe_down_wg<LPR, BPL, EPW, AL, NW>(blockIdx.x, act, idx, w, dw, de, db, out, a);
+                                                      const float *__restrict__ w, const uint4 *__restrict__ dw,
+                                                      const uint8_t *__restrict__ de, const float *__restrict__ db,
+                                                      float *__restrict__ out, MoeArgs a) {
+  moe_down_wg<LPR, BPL, R, NW>(blockIdx.x, act, idx, w, dw, de, db, out, a);
 }
 
-// LDS the staging copies may take (gfx950: 160 KB a workgroup, 64 KB without the attribute).
-constexpr size_t kMoeStageLds = 128 * 1024;
-
-template <int LPR, int BPL, int EPW, int NW>
-void launch_down_cfg(hipStream_t st, const float *act, const int32_t *idx, const float *w, const void *dw,
-                     const void *de, const float *db, float *out, const MoeArgs &a) {
-  constexpr int RS = 64 / LPR;
-  const size_t lds = (size_t)a.T * a.k * a.I * 4;
-  const dim3 grid((a.H + RS - 1) / RS);
-  if (lds <= kMoeStageLds) {
-    static bool attr = false;  // once per instance: the dynamic LDS past 64 KB
-    if (!attr) {
-      (void)hipFuncSetAttribute((const void *)k_moe_down<LPR, BPL, EPW, true, NW>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMoeStageLds);
-      attr = true;
-    }
-    hipLaunchKernelGGL((k_moe_down<LPR, BPL, EPW, true, NW>), grid, dim3(64 * NW), lds, st, act, idx, w,
-                       (const uint4 *)dw, (const uint8_t *)de, db, out, a);
-  } else {
-    hipLaunchKernelGGL((k_moe_down<LPR, BPL, EPW, false, NW>), grid, dim3(64 * NW), 0, st, act, idx, w,
-                       (const uint4 *)dw, (const uint8_t *)de, db, out, a);
-  }
-}
-
-// The waves of a down workgroup and the experts a wave loads at once, by the chosen (token, expert)
-// slots n = T*k (at most n distinct experts): every slot a wave of its own up to 4 (no load is a
-// padding copy), one a wave for 16 waves up to 32 (16 at once, a second round past 16 distinct
-// experts; at T = 5 30.5-30.8 µs a layer against 31.4 for two a wave in 8 waves, and 31.6 for one in
-// 8), else as many as the registers take.
-template <int LPR, int BPL>
+// The waves of a down workgroup, by the most experts chosen: a wave an expert, up to 8 while the staged
+// activations fit 128 KB of LDS; 16 for short rows while the grid is one workgroup a CU (a layer of 5 tokens:
+// 21.4 µs, with 8 waves 22.8; of 3: 15.3 and 16.8).
+template <int LPR, int BPL, int R>
 void launch_down(hipStream_t st, const float *act, const int32_t *idx, const float *w, const void *dw, const void *de,
                  const float *db, float *out, const MoeArgs &a) {
-  const uint32_t n = a.T * a.k;
-  if (n <= 4)
-    launch_down_cfg<LPR, BPL, 1, 4>(st, act, idx, w, dw, de, db, out, a);
-  else if (n <= 32)
-    launch_down_cfg<LPR, BPL, 1, 16>(st, act, idx, w, dw, de, db, out, a);
-  else
-    launch_down_cfg<LPR, BPL, BPL <= 1 ? 8 : 12 / BPL, 8>(st, act, idx, w, dw, de, db, out, a);
+  constexpr int RS = R * 64 / LPR;
+  const dim3 grid((a.H + RS - 1) / RS);
+  const uint32_t n = a.T * a.k < a.E ? a.T * a.k : a.E;
+#define HWK_DN(NW)                                                                                             \
+  hipLaunchKernelGGL((k_moe_down<LPR, BPL, R, NW>), grid, dim3(64 * NW), 0, st, act, idx, w, (const uint4 *)dw, \
+                     (const uint8_t *)de, db, out, a)
+  if constexpr (LPR == 8) {
+    if (n > 8 && a.H <= 256 * RS) {
+      HWK_DN(16);
+      return;
+    }
+  }
+  if constexpr (DownCfg<LPR, BPL, R, 8>::kActs * 8 <= 128 * 1024) {
+    if (n > 4) {
+      HWK_DN(8);
+      return;
+    }
+  }
+  HWK_DN(4);
+#undef HWK_DN
 }
 
 char *check_params(const char *what, const hwk_moe_params *p) {
@@ -105,30 +93,41 @@ MoeArgs args_of(const hwk_moe_params *p) {
   a.norm = (int)p->norm;
   a.scale = hwk::f32_of_bits(p->scale_bits);
   a.mode = (int)p->out_mode;
+  a.span = 1;
   return a;
 }
 
 template <int PPW, bool ROUTE>
 void launch_gate_up(hipStream_t st, const void *x, const float *logits, const float *rbias, int32_t *idx, float *w,
-                    const void *gu_w, const void *gu_e, const float *gu_b, float *act, const MoeArgs &a) {
-  const uint32_t unique_max = a.T * a.k < a.E ? a.T * a.k : a.E;
+                    const void *gu_w, const void *gu_e, const float *gu_b, float *act, MoeArgs a) {
+  const uint32_t unique_max = a.T * a.k < a.E ? a.T * a.k : a.E, nb = a.H / 32;
+  // tiles a workgroup: one until the grid has twice what the chip holds (four workgroups a CU), then as many as
+  // leave that, so that the choice, x and the gated unit are shared by more rows (a layer of 8 tokens of 64
+  // experts at k = 8, I = 1,408: 110 µs with one tile a workgroup, 74 with 8; goals of 512 and 2,048: 74 and 83)
+  const uint32_t wgs = gate_up_wgs(a.I, 4 * PPW) * unique_max, goal = 4 * 256;
+  a.span = wgs < 2 * goal ? 1 : wgs / goal < kMoeSpan ? wgs / goal : kMoeSpan;
   // with the route folded in, one more column of workgroups: the route's own (moe_gate_up_wg)
-  const dim3 g1((a.I + 4 * PPW - 1) / (4 * PPW) + (ROUTE ? 1 : 0), unique_max);
-  const int bpl1 = (int)((a.H / 32 + 63) / 64);
-#define HWK_GU(B)                                                                                         \
-  hipLaunchKernelGGL((k_moe_gate_up<B, PPW, ROUTE>), g1, dim3(256), 0, st, (const uint4 *)x, logits, rbias, idx, w, \
-                     (const uint4 *)gu_w, (const uint8_t *)gu_e, gu_b, act, a)
-  switch (bpl1) {
-    case 1: HWK_GU(1); break;
-    case 2: HWK_GU(2); break;
-    case 3: HWK_GU(3); break;
-    default: HWK_GU(4); break;
-  }
+  const dim3 g1(gate_up_wgs(a.I, 4 * PPW * a.span) + (ROUTE ? 1 : 0), unique_max);
+  // the attribute: dynamic LDS past 64 KB (8 tokens of H = 8,192 take 128 KB)
+#define HWK_GU(L, B)                                                                                              \
+  do {                                                                                                            \
+    static const hipError_t attr = hipFuncSetAttribute((const void *)k_moe_gate_up<L, B, PPW, ROUTE>,             \
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);   \
+    (void)attr;                                                                                                   \
+    hipLaunchKernelGGL((k_moe_gate_up<L, B, PPW, ROUTE>), g1, dim3(256), a.T * x_bytes(a.H), st, (const uint4 *)x, \
+                       logits, rbias, idx, w, (const uint4 *)gu_w, (const uint8_t *)gu_e, gu_b, act, a);          \
+  } while (0)
+  // lanes a row: 32 up to H = 4,096 (a row sum is then half the steps, and one load takes gate and up)
+  if (nb <= 32) HWK_GU(32, 1);
+  else if (nb <= 64) HWK_GU(32, 2);
+  else if (nb <= 96) HWK_GU(32, 3);
+  else if (nb <= 128) HWK_GU(32, 4);
+  else if (nb <= 192) HWK_GU(64, 3);
+  else HWK_GU(64, 4);
 #undef HWK_GU
 }
 
-// K5b: gate_up (with the route folded in when ROUTE), then down with the ordered combine. Past 2
-// tokens a workgroup takes 4 row pairs a wave instead of 2: fewer waves repeat the per-token work.
+// K5b: gate_up (with the route folded in when ROUTE), then down with the ordered combine.
 template <bool ROUTE>
 char *run_experts(hipStream_t st, const void *x, const float *logits, const float *rbias, int32_t *idx, float *w,
                   const void *gu_w, const void *gu_e, const float *gu_b, const void *dn_w, const void *dn_e,
@@ -138,22 +137,29 @@ char *run_experts(hipStream_t st, const void *x, const float *logits, const floa
   else
     launch_gate_up<4, ROUTE>(st, x, logits, rbias, idx, w, gu_w, gu_e, gu_b, act, a);
   if (char *err = hwk::launched(what)) return err;
-  // down: lanes a row by I/32 blocks, the fewest idle slots (8 lanes x 3 blocks for I = 768)
+  // down: lanes a row by I/32 blocks, the fewest idle slots (8 lanes x 3 blocks for I = 768), and row sets enough
+  // that a workgroup has 8 rows to share the staged activations
   const uint32_t nbi = a.I / 32;
-  if (nbi <= 8) launch_down<8, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
-  else if (nbi <= 16) launch_down<16, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
-  else if (nbi <= 24) launch_down<8, 3>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
-  else if (nbi <= 32) launch_down<32, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
-  else if (nbi <= 64) launch_down<64, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
-  else if (nbi <= 128) launch_down<64, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
-  else if (nbi <= 192) launch_down<64, 3>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
-  else launch_down<64, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  if (nbi <= 8) launch_down<8, 1, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 16) launch_down<8, 2, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 24) launch_down<8, 3, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 32) launch_down<16, 2, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 48) launch_down<16, 3, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 64) launch_down<32, 2, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 96) launch_down<32, 3, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 128) launch_down<64, 2, 8>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 192) launch_down<64, 3, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else launch_down<64, 4, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   return hwk::launched(what);
 }
 
-// Tokens up to which hwk_moe_layer folds the route into the gate_up launch: every workgroup routes
-// every token, which past a few tokens costs more vector issue than the route launch it saves.
-constexpr uint32_t kFoldRouteMaxTokens = 2;
+// Whether hwk_moe_layer folds the route into the gate_up launch: up to 2 tokens always, and up to 5 where the
+// choice can be read off the logits (k wave maxima a token and wave; Choose in every workgroup costs more than
+// the launch it saves). A layer of 3, 4, 5, 6 and 8 tokens folded against a route launch, µs: 15.3 and 18.2,
+// 22.9 and 26.6 (k = 8 of 64), 21.4 and 22.8, 43.4 and 43.3 (k = 8), 30.9 and 28.7.
+bool folds_route(const hwk_moe_params *p, const void *router_bias) {
+  return p->tokens <= 2 || (p->tokens <= 5 && p->score == HWK_SCORE_SOFTMAX && !router_bias);
+}
 
 }  // namespace
 
@@ -207,7 +213,7 @@ HWK_API char *hwk_moe_layer(void *stream, const void *x, const void *logits, con
             workspace_bytes, hwk_moe_workspace_bytes(p));
   const MoeArgs a = args_of(p);
   hipStream_t st = (hipStream_t)stream;
-  if (p->tokens <= kFoldRouteMaxTokens)
+  if (folds_route(p, router_bias))
     return run_experts<true>(st, x, (const float *)logits, (const float *)router_bias, (int32_t *)idx, (float *)w,
                              gu_w, gu_e, (const float *)gu_b, dn_w, dn_e, (const float *)dn_b, (float *)out,
                              (float *)workspace, a, "hwk_moe_layer");

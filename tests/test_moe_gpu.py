@@ -235,3 +235,47 @@ def test_moe_layer_small_shapes_sigmoid(dev, orc):
         assert np.all(ulp_diff(w.cpu().numpy()[t], ow) <= 1)
     want = orc.experts(x.cpu().numpy().astype(np.float32), *_np(idx, w, gw, ge, dw, de))
     check_close(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize(
+    "T,E,k,H,I",
+    [
+        (5, 8, 2, 1024, 32),      # one block a row of down, 32 lanes a row of gate_up with a block each
+        (8, 16, 8, 2080, 512),    # the last block of a lane past the row, n = 64 choices of 16 experts
+        (3, 32, 4, 2912, 1024),   # 16 lanes a row
+        (5, 16, 2, 4096, 1504),   # 47 of 48 blocks
+        (4, 8, 4, 4128, 2016),    # 64 lanes a row of gate_up, 32 of down
+        (2, 4, 2, 8192, 3072),    # the widest x
+        (8, 4, 1, 256, 4096),     # 64 lanes a row of down; every token on a few experts
+        (3, 3, 3, 512, 6112),     # 191 of 192 blocks, every expert by every token
+        (1, 2, 1, 96, 8192),      # the longest rows of down
+        (8, 64, 8, 1024, 4064),   # several tiles a workgroup of gate_up, the last workgroup's past I
+    ],
+)
+def test_moe_layer_tiles(dev, orc, T, E, k, H, I):
+    """Each layout of gate_up (by H) and of down (by I) at its edges, the route folded in: idx as the
+    oracle's Choose, the output as the oracle's experts'; hwk_moe_experts with an id out of range and a
+    repeated one (neither counts a second time)."""
+    print(f"moe layer T={T} E={E} k={k} H={H} I={I}", flush=True)
+    x, logits, gw, ge, dw, de = experts_case(T, E, H, I, name="tiles")
+    out, idx, w = ops.moe_layer(x, logits, k, gw, ge, dw, de)
+    lg, ii, ww = _np(logits, idx, w)
+    for t in range(T):
+        oi, ow = orc.choose(lg[t], k)
+        assert np.array_equal(ii[t], oi), (t, ii[t], oi)
+        assert np.all(ulp_diff(ww[t], ow) <= 1)
+    x32, host = x.cpu().numpy().astype(np.float32), _np(gw, ge, dw, de)
+    want = orc.experts(x32, ii, ww, *host)
+    check_close(out.cpu().numpy(), want)
+    if k < 2:
+        return
+    bad = idx.clone()
+    bad[0, 0] = E
+    bad[T - 1, k - 1] = bad[T - 1, 0] if T > 1 else -1
+    wz, i2 = ww.copy(), bad.cpu().numpy()
+    wz[0, 0] = 0.0
+    if T > 1 or k > 1:
+        wz[T - 1, k - 1] = 0.0
+    i2 = np.where(wz == 0.0, ii, i2)  # for the oracle: a valid id of weight zero
+    got = ops.moe_experts(x, bad, w, gw, ge, dw, de)
+    check_close(got.cpu().numpy(), orc.experts(x32, i2, wz, *host))
