@@ -172,7 +172,7 @@ _lib = None
 
 
 class _Lib:
-    """The loaded library: attribute access gives a checked Python callable per entry point."""
+    """The loaded library: an attribute per entry point, a checked Python callable."""
 
     def __init__(self, path: str):
         self.path = path
@@ -185,15 +185,15 @@ class _Lib:
         if abi != ABI:
             raise HwkLibraryError(f"{path}: ABI {abi}, this binding speaks {ABI}")
 
+        # a checked callable per entry point, made once: made anew at each access they cost more than the call
+        for name, (res, _) in SIGNATURES.items():
+            fn = getattr(self._cdll, name)
+            setattr(self, name, self._checked(name, fn) if res == ERR else fn)
+
     def raw(self, name: str):
         return getattr(self._cdll, name)
 
-    def __getattr__(self, name: str):
-        if name not in SIGNATURES:
-            raise AttributeError(name)
-        fn = getattr(self._cdll, name)
-        if SIGNATURES[name][0] != ERR:
-            return fn
+    def _checked(self, name: str, fn):
         free = self._cdll.hwk_free_error
 
         def call(*args):
@@ -210,6 +210,9 @@ class _Lib:
 def load(path: str | None = None) -> _Lib:
     """The process's libhwk; raises HwkLibraryError when it is missing or of another ABI."""
     global _lib
+    lib = _lib
+    if lib is not None and path is None:  # published whole: no lock
+        return lib
     with _lock:
         if _lib is not None and (path is None or path == _lib.path):
             return _lib

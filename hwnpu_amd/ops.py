@@ -18,11 +18,16 @@ OUT_MODES = {"f32": hwk.OUT_F32, "f16": hwk.OUT_F16, "add": hwk.OUT_ADD_F32, "sw
 
 def f32_bits(v: float) -> int:
     """A float32 scalar as the uint32 bit pattern the ABI takes."""
-    return struct.unpack("<I", struct.pack("<f", float(v)))[0]
+    return _U32.unpack(_F32.pack(float(v)))[0]
+
+
+_U32, _F32 = struct.Struct("<I"), struct.Struct("<f")
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the current stream of the current device as torch keeps it; torch.cuda.current_stream() makes a Stream
+    # object for it, 2 µs a call
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _need(t: torch.Tensor, name: str, dtype, shape=None):
@@ -34,7 +39,7 @@ def _need(t: torch.Tensor, name: str, dtype, shape=None):
         raise TypeError(f"{name}: dtype {t.dtype}, want {dtype}")
     if not t.is_contiguous():
         raise ValueError(f"{name}: must be contiguous")
-    if shape is not None and tuple(t.shape) != tuple(shape):
+    if shape is not None and t.shape != shape:
         raise ValueError(f"{name}: shape {tuple(t.shape)}, want {tuple(shape)}")
 
 
@@ -171,13 +176,8 @@ def mxfp4_encode(x: torch.Tensor):
 
 def attn_params(heads, kv_heads, length, capacity, kv_int8=False, scale=None, out_mode="f32", split=0,
                 head_dim=128):
-    p = hwk.AttnParams()
-    p.heads, p.kv_heads, p.head_dim = heads, kv_heads, head_dim
-    p.len, p.capacity, p.kv_int8 = length, capacity, 1 if kv_int8 else 0
-    p.scale_bits = f32_bits(head_dim ** -0.5 if scale is None else scale)
-    p.out_mode = OUT_MODES[out_mode]
-    p.split = split
-    return p
+    return hwk.AttnParams(heads, kv_heads, head_dim, length, capacity, 1 if kv_int8 else 0,
+                          f32_bits(head_dim ** -0.5 if scale is None else scale), OUT_MODES[out_mode], split)
 
 
 def attn_workspace(p) -> torch.Tensor:
@@ -304,14 +304,9 @@ def moe_route(logits, k, score="softmax", norm=True, scale=0.0, bias=None):
 def _moe_params(T, H, I, E, k, out_mode, act, alpha, limit, score="softmax", norm=True, scale=0.0):
     if act not in ("silu", "gptoss"):
         raise ValueError(f"act {act!r}: 'silu' or 'gptoss'")
-    p = hwk.MoeParams()
-    p.tokens, p.hidden, p.inter, p.experts, p.k = T, H, I, E, k
-    p.out_mode = OUT_MODES[out_mode]
-    p.act = hwk.ACT_SILU if act == "silu" else hwk.ACT_GPTOSS
-    p.alpha_bits, p.limit_bits = f32_bits(alpha), f32_bits(limit)
-    p.score = hwk.SCORE_SOFTMAX if score == "softmax" else hwk.SCORE_SIGMOID
-    p.norm, p.scale_bits = 1 if norm else 0, f32_bits(scale)
-    return p
+    return hwk.MoeParams(T, H, I, E, k, OUT_MODES[out_mode], hwk.ACT_SILU if act == "silu" else hwk.ACT_GPTOSS,
+                         f32_bits(alpha), f32_bits(limit), hwk.SCORE_SOFTMAX if score == "softmax" else hwk.SCORE_SIGMOID,
+                         1 if norm else 0, f32_bits(scale))
 
 
 def _moe_operands(x, gu_w, gu_e, dn_w, dn_e, gu_b, dn_b):
