@@ -87,6 +87,15 @@ __device__ __forceinline__ double wave_sum_f64_all(double v) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// The sum of a double over each row of 16 lanes, in every lane of it (DPP row rotations).
+__device__ __forceinline__ double row16_sum_f64(double v) {
+  v += dpp_f64<0x128, 0xf, false>(v);  // row_ror:8
+  v += dpp_f64<0x124, 0xf, false>(v);  // row_ror:4
+  v += dpp_f64<0x122, 0xf, false>(v);  // row_ror:2
+  v += dpp_f64<0x121, 0xf, false>(v);  // row_ror:1
+  return v;
+}
+
 // Per-head RMSNorm then RoPE of one 128-wide head held as dims (l, l+64) by lane l: (x * r) * w
 // with r = float(1 / sqrt(mean(x^2) + eps)) (mean in float64), then x*cos + rotate_half(x)*sin
 // with the position's float32 tables (rotate_half = cat(-x2, x1); reference internal/llm/blocks/

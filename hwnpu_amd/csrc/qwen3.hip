@@ -36,11 +36,13 @@ using hwk_glue::embed_blocks;
 using hwk_glue::k_embed_ids;
 using hwk_glue::k_silu_mul;
 
-// One wave a (token t, head slot): slots [0, heads) are query heads, [heads, heads+kvh) key heads,
-// then value heads. A lane holds dims l and l+64, the pair rotate_half mixes. q and k: per-head
-// RMSNorm with fp32 weights, then RoPE at position *pos + base + t with the float32 tables
+// 16 lanes a (token t, head slot), 16 slots a workgroup: slots [0, heads) are query heads, [heads, heads+kvh) key
+// heads, then value heads. Lane i of the 16 holds dims 4i .. 4i+3 and 64 more, the pairs rotate_half mixes. q and
+// k: per-head RMSNorm with fp32 weights, then RoPE at position *pos + base + t with the float32 tables
 // (reference internal/llm/blocks/blocks.go:412-445), rounded to fp16; q to q16 (t, heads, 128),
 // k to the cache; v rounded to fp16 into the cache.
+// Bound by the vector ALUs (the float64 sum, square root and quotient) with a wave a head: four heads share
+// them, and memory is read and written 16 and 8 bytes a lane. 1,024 tokens of 32 slots: 9.3 -> 6.3 µs (traced).
 __global__ __launch_bounds__(256) void k_qk_rope(const float *__restrict__ qkv, const float *__restrict__ qn,
                                                  const float *__restrict__ kn, const float *__restrict__ cos_t,
                                                  const float *__restrict__ sin_t, const int32_t *__restrict__ pos,
@@ -48,27 +50,36 @@ __global__ __launch_bounds__(256) void k_qk_rope(const float *__restrict__ qkv, 
                                                  f16 *__restrict__ vc, uint32_t heads, uint32_t kvh, uint32_t cap,
                                                  double eps) {
 #pragma clang fp contract(off)
-  const uint32_t slot = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const uint32_t t = blockIdx.y, l = threadIdx.x & 63;
-  const uint32_t slots = heads + 2 * kvh;
-  if (slot >= slots) return;
+  using hwk_glue::f32x4;
+  using hwk_glue::f16x4;
+  const uint32_t slots = heads + 2 * kvh, first = blockIdx.x * 16 + threadIdx.x / 16;
+  const uint32_t slot = min(first, slots - 1);  // past the last the last again, not stored
+  const uint32_t t = blockIdx.y, i = threadIdx.x & 15;
+  const f32x4 *x = (const f32x4 *)(qkv + ((size_t)t * slots + slot) * 128);
+  const f32x4 *nw = (const f32x4 *)(slot < heads ? qn : kn);
+  const f32x4 x0 = x[i], x1 = x[i + 16], w0 = nw[i], w1 = nw[i + 16];
   const uint32_t p = (uint32_t)*pos + base + t;
-  const float *x = qkv + (size_t)t * slots * 128 + (size_t)slot * 128;
-  float x0 = x[l], x1 = x[l + 64];
-  if (slot >= heads + kvh) {
-    const uint32_t j = slot - heads - kvh;
-    f16 *dst = vc + ((size_t)j * cap + p) * 128;
-    dst[l] = (f16)x0;
-    dst[l + 64] = (f16)x1;
-    return;
+  const f32x4 c = ((const f32x4 *)cos_t)[(size_t)p * 16 + i], s = ((const f32x4 *)sin_t)[(size_t)p * 16 + i];
+  double ss = 0.0;
+#pragma unroll
+  for (int j = 0; j < 4; j++) ss += (double)x0[j] * (double)x0[j] + (double)x1[j] * (double)x1[j];
+  ss = row16_sum_f64(ss);
+  const float r = (float)(1.0 / sqrt(ss / 128.0 + eps));
+  const bool v = slot >= heads + kvh;
+  f16x4 o0, o1;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const float y0 = (x0[j] * r) * w0[j], y1 = (x1[j] * r) * w1[j];
+    const float r0 = f32_value(y0 * c[j] + (-y1) * s[j]), r1 = f32_value(y1 * c[j] + y0 * s[j]);
+    o0[j] = (f16)(v ? x0[j] : r0);
+    o1[j] = (f16)(v ? x1[j] : r1);
   }
-  float o0, o1;
-  const float *nw = slot < heads ? qn : kn;
-  head_norm_rope(x0, x1, nw[l], nw[l + 64], cos_t[(size_t)p * 64 + l], sin_t[(size_t)p * 64 + l], eps, o0, o1);
-  f16 *dst = slot < heads ? q16 + ((size_t)t * heads + slot) * 128
-                          : kc + ((size_t)(slot - heads) * cap + p) * 128;
-  dst[l] = (f16)o0;
-  dst[l + 64] = (f16)o1;
+  if (first >= slots) return;
+  f16 *dst = v              ? vc + ((size_t)(slot - heads - kvh) * cap + p) * 128
+             : slot < heads ? q16 + ((size_t)t * heads + slot) * 128
+                            : kc + ((size_t)(slot - heads) * cap + p) * 128;
+  ((f16x4 *)dst)[i] = o0;
+  ((f16x4 *)dst)[i + 16] = o1;
 }
 
 __global__ void k_set_i32(int32_t *__restrict__ p, int32_t v) { *p = v; }
@@ -433,7 +444,7 @@ char *prefill_piece(hwk_qwen3 *m, hipStream_t st, uint32_t T, uint32_t start, bo
   for (auto &ly : m->L) {
     HWK_Q(hwk::rmsnorm_f16(st, m->h, ly.in_norm, m->eps, m->x16, T, c.hidden));
     HWK_Q(hwk_mxfp4_gemm(st, m->x16, ly.qkv.w, ly.qkv.e, m->qkv, T, m->qkv_n, c.hidden, HWK_OUT_F32));
-    hipLaunchKernelGGL(k_qk_rope, dim3((slots + 3) / 4, T), dim3(256), 0, st, m->qkv, ly.q_norm, ly.k_norm, m->cos_t,
+    hipLaunchKernelGGL(k_qk_rope, dim3((slots + 15) / 16, T), dim3(256), 0, st, m->qkv, ly.q_norm, ly.k_norm, m->cos_t,
                        m->sin_t, m->pos, 0u, m->q16, ly.kc, ly.vc, c.heads, c.kv_heads, c.max_ctx, m->eps);
     HWK_Q(hwk::launched("qwen3 qk_rope"));
     HWK_Q(hwk_attn_prefill_ws(st, m->q16, ly.kc, ly.vc, m->att16, m->ws, m->ws_bytes, T, start, &pp));
@@ -482,7 +493,7 @@ char *verify_piece(hwk_qwen3 *m, hipStream_t st, uint32_t T, uint32_t start) {
   for (auto &ly : m->L) {
     HWK_Q(hwk::rmsnorm_f16(st, m->h, ly.in_norm, m->eps, m->x16, T, c.hidden));
     HWK_Q(rows_linear(st, m->x16, ly.qkv, m->qkv, T, HWK_OUT_F32));
-    hipLaunchKernelGGL(k_qk_rope, dim3((slots + 3) / 4, T), dim3(256), 0, st, m->qkv, ly.q_norm, ly.k_norm, m->cos_t,
+    hipLaunchKernelGGL(k_qk_rope, dim3((slots + 15) / 16, T), dim3(256), 0, st, m->qkv, ly.q_norm, ly.k_norm, m->cos_t,
                        m->sin_t, m->pos, 0u, m->q16, ly.kc, ly.vc, c.heads, c.kv_heads, c.max_ctx, m->eps);
     HWK_Q(hwk::launched("qwen3 verify qk_rope"));
     HWK_Q(hwk_attn_prefill_ws(st, m->q16, ly.kc, ly.vc, m->att16, m->ws, m->ws_bytes, T, start, &pp));
