@@ -126,26 +126,28 @@ void dispatch(hipStream_t st, const void *w, const void *s, const void *x, void 
 
 // K7r: Y (T, n) = X W^T for fp16 W (n, k) and T <= 8 fp16 vectors X (T, k): the tied head over the
 // rows of a speculative verify, each weight row read once for all T vectors. The workgroup copies X
-// into LDS; a wave walks rows (grid-stride), 64 lanes over a row's 16-byte chunks, 4 chunks a lane
-// a pass, and with a single pass (k <= 2048) the next row's chunks are loaded before this row's
-// products.
-template <int TT, bool ONEPASS>
+// into LDS; a wave walks sets of R rows (grid-stride), 64 lanes over a row's 16-byte chunks, 4 chunks a
+// lane a pass, and with a single pass (k <= 2048) the next set's chunks are loaded before this set's
+// products. Past 3 vectors the reads of X from LDS and the products bound it: a read of X serves both rows of a
+// set, and the two rows' sums share their steps (5 vectors, 151,936 rows of
+// 2,048, launches back to back: 132 -> 120 µs; 8: 162 -> 140; 8 against 32,768 of 4,096: 88 -> 67).
+template <int TT, bool ONEPASS, int R>
 __global__ __launch_bounds__(256) void k_f16_gemv_rows(const uint4 *__restrict__ w, const uint4 *__restrict__ x,
                                                        void *__restrict__ y, uint32_t n, uint32_t nc, int mode) {
   extern __shared__ uint4 xsr[];  // (TT, nc)
   const int lane = threadIdx.x & 63;
-  const uint32_t waves = gridDim.x * 4;
-  uint32_t r = blockIdx.x * 4 + (threadIdx.x >> 6);
-  // every load issued unconditionally (a chunk past nc reads the last one; dot4 skips it): a load
-  // under a branch is waited for where the branches join
-  auto load4 = [&](uint32_t row, uint32_t base, uint4 (&c)[4]) {
+  const uint32_t step = gridDim.x * 4 * R;
+  uint32_t r = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
+  // every load issued unconditionally (a row past n reads the last one, a chunk past nc the last one; dot4
+  // skips it): a load under a branch is waited for where the branches join
+  auto load4 = [&](uint32_t row, uint32_t base, uint4 (&c)[R][4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const uint32_t ch = min(base + j * 64 + lane, nc - 1);
-      c[j] = load_stream(&w[(size_t)row * nc + ch]);
-    }
+    for (int i = 0; i < R; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        c[i][j] = load_stream(&w[(size_t)min(row + i, n - 1) * nc + min(base + j * 64 + lane, nc - 1)]);
   };
-  // x's chunks (up to 8 a thread) loaded first, then the first row's weights (single pass), then x
+  // x's chunks (up to 8 a thread) loaded first, then the first rows' weights (single pass), then x
   // written to LDS waiting on x only (past x's end the last chunk again, into its own slot)
   constexpr int XF = TT < 8 ? TT : 8;
   const uint32_t xn = TT * nc;
@@ -153,69 +155,90 @@ __global__ __launch_bounds__(256) void k_f16_gemv_rows(const uint4 *__restrict__
 #pragma unroll
   for (int j = 0; j < XF; j++) xv[j] = x[min((uint32_t)(threadIdx.x + j * 256), xn - 1)];
   issue_order();
-  uint4 cur[4];
-  if constexpr (ONEPASS) load4(min(r, n - 1), 0, cur);
+  uint4 cur[R][4];
+  if constexpr (ONEPASS) load4(r, 0, cur);
   issue_order();
 #pragma unroll
   for (int j = 0; j < XF; j++) xsr[min((uint32_t)(threadIdx.x + j * 256), xn - 1)] = xv[j];
   for (uint32_t i = threadIdx.x + XF * 256; i < xn; i += 256) xsr[i] = x[i];
   __syncthreads();
-  auto dot4 = [&](const uint4 (&c)[4], uint32_t base, float (&acc)[TT]) {
+  auto dot4 = [&](const uint4 (&c)[R][4], uint32_t base, float (&acc)[R][TT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const uint32_t ch = base + j * 64 + lane;
       if (ch >= nc) continue;
-      const uint32_t cw[4] = {c[j].x, c[j].y, c[j].z, c[j].w};
 #pragma unroll
       for (int v = 0; v < TT; v++) {
-        const uint4 xv = xsr[(size_t)v * nc + ch];
-        const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
-        float d0 = 0.0f, d1 = 0.0f;
-        d0 = __builtin_amdgcn_fdot2(h2_of_bits(cw[0]), h2_of_bits(xw[0]), d0, false);
-        d1 = __builtin_amdgcn_fdot2(h2_of_bits(cw[1]), h2_of_bits(xw[1]), d1, false);
-        d0 = __builtin_amdgcn_fdot2(h2_of_bits(cw[2]), h2_of_bits(xw[2]), d0, false);
-        d1 = __builtin_amdgcn_fdot2(h2_of_bits(cw[3]), h2_of_bits(xw[3]), d1, false);
-        acc[v] += d0 + d1;
+        const uint4 xc = xsr[(size_t)v * nc + ch];
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+          float d0 = __builtin_amdgcn_fdot2(h2_of_bits(c[i][j].x), h2_of_bits(xc.x), 0.0f, false);
+          float d1 = __builtin_amdgcn_fdot2(h2_of_bits(c[i][j].y), h2_of_bits(xc.y), 0.0f, false);
+          d0 = __builtin_amdgcn_fdot2(h2_of_bits(c[i][j].z), h2_of_bits(xc.z), d0, false);
+          d1 = __builtin_amdgcn_fdot2(h2_of_bits(c[i][j].w), h2_of_bits(xc.w), d1, false);
+          acc[i][v] += d0 + d1;
+        }
       }
     }
   };
-  if (r >= n) return;
-  for (; r < n; r += waves) {
-    float acc[TT];
+  for (; r < n; r += step) {
+    float acc[R][TT];
 #pragma unroll
-    for (int v = 0; v < TT; v++) acc[v] = 0.0f;
+    for (int i = 0; i < R; i++)
+#pragma unroll
+      for (int v = 0; v < TT; v++) acc[i][v] = 0.0f;
     if constexpr (ONEPASS) {
-      uint4 nxt[4];
-      const uint32_t rn = r + waves < n ? r + waves : r;
-      load4(rn, 0, nxt);
+      uint4 nxt[R][4];
+      load4(r + step < n ? r + step : r, 0, nxt);
       dot4(cur, 0, acc);
 #pragma unroll
-      for (int j = 0; j < 4; j++) cur[j] = nxt[j];
+      for (int i = 0; i < R; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) cur[i][j] = nxt[i][j];
     } else {
       for (uint32_t base = 0; base < nc; base += 256) {
-        uint4 c[4];
+        uint4 c[R][4];
         load4(r, base, c);
         dot4(c, base, acc);
       }
     }
 #pragma unroll
     for (int v = 0; v < TT; v++) {
-      const float s = group_sum<64>(acc[v]);
-      if (lane == 0) store_out(y, (size_t)v * n + r, s, mode);
+      if constexpr (R == 2) {
+        // the two rows' sums at once: each half of the wave adds the other half's part of its row
+        swap_rows32(acc[0][v], acc[1][v]);
+        const float s = group_sum<32>(acc[0][v] + acc[1][v]);
+        if ((lane & 31) == 0 && r + (lane >> 5) < n) store_out(y, (size_t)v * n + r + (lane >> 5), s, mode);
+      } else {
+        const float s = group_sum<64>(acc[0][v]);
+        if (lane == 0) store_out(y, (size_t)v * n + r, s, mode);
+      }
     }
   }
 }
 
-template <int TT>
-void launch_f16_rows(hipStream_t st, const void *w, const void *x, void *y, uint32_t n, uint32_t nc, int mode) {
-  const uint32_t blocks = (n + 3) / 4 < 1024u ? (n + 3) / 4 : 1024u;
+template <int TT, int R>
+void launch_f16_rows_of(hipStream_t st, const void *w, const void *x, void *y, uint32_t n, uint32_t nc, int mode) {
+  const uint32_t sets = (n + 4 * R - 1) / (4 * R), blocks = sets < 1024u ? sets : 1024u;
   const size_t lds = (size_t)TT * nc * 16;
   if (nc <= 256)
-    hipLaunchKernelGGL((k_f16_gemv_rows<TT, true>), dim3(blocks), dim3(256), lds, st, (const uint4 *)w,
+    hipLaunchKernelGGL((k_f16_gemv_rows<TT, true, R>), dim3(blocks), dim3(256), lds, st, (const uint4 *)w,
                        (const uint4 *)x, y, n, nc, mode);
   else
-    hipLaunchKernelGGL((k_f16_gemv_rows<TT, false>), dim3(blocks), dim3(256), lds, st, (const uint4 *)w,
+    hipLaunchKernelGGL((k_f16_gemv_rows<TT, false, R>), dim3(blocks), dim3(256), lds, st, (const uint4 *)w,
                        (const uint4 *)x, y, n, nc, mode);
+}
+
+// Two rows a wave for 4 vectors and more, once the waves walk several sets (k <= 2048) or a row is several
+// passes: 5 vectors against 16,384 rows of 2,048 17.5 µs (one row a wave: 16.3), 32,768 28.0 (28.2), 151,936 120
+// (132); 4 against 2,048 rows of 8,192 11.6 (10.3), 4,096 16.0 (19.8). Up to 3 vectors the loads bound either
+// (3 against 151,936: 103.6 and 103.8). Four rows a wave hold too many registers (slower than two throughout).
+template <int TT>
+void launch_f16_rows(hipStream_t st, const void *w, const void *x, void *y, uint32_t n, uint32_t nc, int mode) {
+  if constexpr (TT >= 4) {
+    if (n >= (nc <= 256 ? 32768u : 4096u)) return launch_f16_rows_of<TT, 2>(st, w, x, y, n, nc, mode);
+  }
+  launch_f16_rows_of<TT, 1>(st, w, x, y, n, nc, mode);
 }
 
 }  // namespace

@@ -192,6 +192,22 @@ def test_f16_gemv_rows_parity(dev, orc, T, n, k):
     check_close(one, y32[T - 1], tol=1e-5)
 
 
+# two rows a wave: an odd row count (the last set's second row is past the end), a last chunk past the row, rows of
+# several passes, the fewest and the most vectors, and the row counts just below (one row a wave)
+@pytest.mark.parametrize("T,n,k", [(4, 32769, 512), (8, 32771, 2048), (6, 32767, 264), (4, 4097, 2056), (8, 4096, 4096),
+                                   (5, 4095, 2560), (4, 4099, 8192)])
+@pytest.mark.parametrize("mode", ["f32", "add"])
+def test_f16_gemv_rows_two_a_wave(dev, orc, T, n, k, mode):
+    print(f"f16_gemv_rows T={T} n={n} k={k} {mode}", flush=True)
+    w = synth.normal(n * k, f"k7r2.{n}.{k}", std=0.02).view(n, k)
+    x = synth.normal(T * k, f"k7r2.{T}.{n}.{k}.x").view(T, k)
+    want = orc.sgemm(x.cpu().numpy().astype(np.float32), w.cpu().numpy().astype(np.float32), transb=True)
+    y = torch.ones((T, n), dtype=torch.float32, device="cuda") if mode == "add" else None
+    got = ops.f16_gemv_rows(w, x, mode, y).cpu().numpy()
+    for t in range(T):
+        check_close(got[t], want[t] + (1.0 if mode == "add" else 0.0))
+
+
 # ---------------- K1r: several vectors, weights read once ----------------
 
 # (T >= 6 with k a multiple of 512: the matrix-core form; the rest: the VALU form)
