@@ -925,10 +925,12 @@ namespace {
 
 // The decode-step GEMV's workgroups: 8 waves of 2 rows a pass (x is made once for 8 waves' rows, and
 // the model's shapes still give every CU whole workgroups: qkv 2048 row sets, 256 workgroups;
-// gate_up 6144, 768; measured against 4 and 16 waves, and 4 rows a pass).
+// gate_up 6144, 768; measured against 4 and 16 waves, and 4 rows a pass). The merging GEMV takes one row a
+// wave, 256 workgroups for the model's 2,048 rows: with two it leaves half the CUs idle (8 decode steps behind
+// 1,024 positions 5,386 -> 5,341 µs; 16 waves of one row: 5,614).
 template <int BPL, int XM, bool SWIGLU, int MODE>
 void launch_x(hipStream_t st, const void *w, const void *e, const XIn &in, void *y, uint32_t n, uint32_t nb) {
-  constexpr int WPB = 8, RPW = 2;
+  constexpr int WPB = 8, RPW = XM == X_MERGE && !SWIGLU ? 1 : 2;
   const uint32_t sets = (n + RPW - 1) / RPW;
   const void *xa = XM == X_F16 ? (const void *)in.x16 : XM == X_NORM ? (const void *)in.h : (const void *)in.ws;
 #define HWK_XL(MBC) hipLaunchKernelGGL((k_mxfp4_gemv_x<BPL, RPW, XM, SWIGLU, WPB, MODE, MBC>), dim3((sets + WPB - 1) / WPB), \
