@@ -112,6 +112,22 @@ def test_attn_decode_int8(dev, orc, heads, kvh, L):
     check_close(got, want)
 
 
+# full tiles without key masks, then the last ones with them: the length a multiple of a wave's keys (128), one more,
+# one less, a tile's edge; maxima that rise along the keys (every tile rescales), fall (none after the first), and
+# NaN in the rows past the length
+@pytest.mark.parametrize("L", [512, 513, 511, 1024 - 48, 1024 - 49])
+@pytest.mark.parametrize("heads,slope", [(32, 1.0), (16, -1.0), (8, 0.0)])
+def test_attn_decode_full_tiles(dev, orc, heads, slope, L):
+    print(f"attn full tiles heads={heads} slope={slope} L={L}", flush=True)
+    q, k, v = case(heads, 8, L, 1024, f"c3.full.{heads}")
+    ramp = torch.linspace(0.0, slope, 1024, device="cuda").view(1, 1024, 1)
+    k = (k.float() + ramp * q.float().mean(0).sign()).half()
+    k[:, L:], v[:, L:] = float("nan"), float("nan")
+    want = orc.attn_decode(q.cpu().numpy().astype(np.float32), k[:, :L].cpu().numpy().astype(np.float32),
+                           v[:, :L].cpu().numpy().astype(np.float32), 1 / math.sqrt(128))
+    check_close(ops.attn_decode(q, k, v, L, split=512).cpu().numpy(), want)
+
+
 def test_attn_decode_empty_is_zero(dev):
     q, k, v = case(32, 8, 0, 16, "c3.empty")
     got = ops.attn_decode(q, k, v, 0).cpu().numpy()
