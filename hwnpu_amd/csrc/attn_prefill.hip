@@ -380,8 +380,10 @@ __global__ __launch_bounds__(256 * S) __attribute__((amdgpu_waves_per_eu(3))) vo
   }
 }
 
-// The chunks' states of each row whose keys were split, merged (paged.go:252-310 in base 2): one wave a row,
-// lane c holding chunk c's m and l (at most 64 chunks), then two dims a lane, eight chunks' loads at once.
+// The chunks' states of each row whose keys were split, merged: one wave a row, lane c holding chunk c's m and l
+// (at most 64 chunks), then two dims a lane, eight chunks' loads at once. A chunk none of whose keys the row saw (l
+// exactly 0) adds nothing; every other one is weighed by 2^(m - top), its NaN or infinite l or O included, so that a
+// NaN or +Inf score makes the row NaN as it does in one workgroup's sums.
 constexpr uint32_t kMaxSplit = 64;
 __global__ __launch_bounds__(256) void k_attn_prefill_merge(const float *__restrict__ ws, void *__restrict__ out,
                                                             PrefillArgs a) {
@@ -394,10 +396,11 @@ __global__ __launch_bounds__(256) void k_attn_prefill_merge(const float *__restr
   const float *part = ws + (size_t)b * a.cut.chunks * kPart;
   const uint32_t cl = min(lane, chunks - 1);
   const float mc = part[cl * kPart + kRows * 128 + rw], lc = part[cl * kPart + kRows * 129 + rw];
-  const bool some = lane < chunks && lc > 0.0f;
+  const bool some = lane < chunks && lc != 0.0f;
+  const uint64_t seen = __ballot(some);
   const float top = group_max_dpp<64>(some ? mc : -__builtin_inff());
   const float w = some ? exp2f(mc - top) : 0.0f;
-  const float den = group_sum<64>(w * (some ? lc : 0.0f));
+  const float den = group_sum<64>(some ? w * lc : 0.0f);
   float n0 = 0.0f, n1 = 0.0f;
   for (uint32_t c0 = 0; c0 < chunks; c0 += 8) {
     float2 o[8];
@@ -406,14 +409,15 @@ __global__ __launch_bounds__(256) void k_attn_prefill_merge(const float *__restr
       o[u] = *(const float2 *)(part + (size_t)min(c0 + u, chunks - 1) * kPart + rw * 128 + 2 * lane);
 #pragma unroll
     for (int u = 0; u < 8; u++) {
-      const float wc = c0 + u < chunks ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), (int)(c0 + u))) : 0.0f;
-      n0 += wc > 0.0f ? wc * o[u].x : 0.0f;
-      n1 += wc > 0.0f ? wc * o[u].y : 0.0f;
+      const float wc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), (int)(c0 + u)));
+      const bool add = (seen >> (c0 + u)) & 1;  // (c0 + u < 64; lanes past the chunks saw nothing)
+      n0 += add ? wc * o[u].x : 0.0f;
+      n1 += add ? wc * o[u].y : 0.0f;
     }
   }
   const size_t o0 = ((size_t)t * a.heads + (h << a.gs) + (row & ((1u << a.gs) - 1))) * 128 + 2 * lane;
-  store_out(out, o0, den > 0.0f ? n0 / den : 0.0f, a.mode);
-  store_out(out, o0 + 1, den > 0.0f ? n1 / den : 0.0f, a.mode);
+  store_out(out, o0, den == 0.0f ? 0.0f : n0 / den, a.mode);
+  store_out(out, o0 + 1, den == 0.0f ? 0.0f : n1 / den, a.mode);
 }
 
 // How the rows of `tokens` positions from start on are cut. Unsplit (no workspace) a chunk is all of a

@@ -281,6 +281,44 @@ def test_attn_prefill_workspace_checked(dev):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("bad", [math.nan, math.inf, -math.inf])
+@pytest.mark.parametrize("heads,kvh,T,start,key", [
+    (16, 8, 5, 1024, 3), (16, 8, 5, 1024, 1026), (32, 8, 33, 1500, 700),  # split
+    (4, 2, 20, 60, 10), (4, 2, 40, 90, 100), (8, 8, 70, 300, 200)])       # one, two and three key groups
+def test_attn_prefill_non_finite_key(dev, heads, kvh, T, start, key, bad):
+    """One NaN or infinite value in a key: the rows that see it are NaN where the float64 softmax is (a NaN score, or
+    one of +Inf) and leave the key out where its score is -Inf; the rows before it do not change. The same with the
+    keys split over workgroups as without; bound as in test_attn_prefill_scales."""
+    from hwnpu_amd import hwk
+
+    print(f"attn prefill non-finite key={key} bad={bad} heads={heads} kv={kvh} T={T} start={start}", flush=True)
+    cap = start + T
+    name = f"c3n.{heads}.{T}.{start}"
+    q = synth.normal(T * heads * 128, name + ".q").view(T, heads, 128)
+    k = synth.normal(kvh * cap * 128, name + ".k").view(kvh, cap, 128)
+    v = synth.normal(kvh * cap * 128, name + ".v").view(kvh, cap, 128)
+    k[kvh - 1, key, 77] = bad
+    p = ops.attn_params(heads, kvh, cap, cap)
+    assert (hwk.load().hwk_attn_prefill_workspace_bytes(T, start, p) > 0) == (start >= 1000)
+    got = ops.attn_prefill(q, k, v, start, out_mode="f32").cpu().double()
+    whole = torch.empty((T, heads, 128), dtype=torch.float32, device="cuda")
+    hwk.load().hwk_attn_prefill(ops._stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(), whole.data_ptr(), T, start, p)
+    whole = whole.cpu().double()
+    qd, kd, vd = q.cpu().double(), k.cpu().double(), v.cpu().double()
+    see = torch.arange(cap)[None] <= start + torch.arange(T)[:, None]
+    lost = 0
+    for h in range(heads):
+        s = qd[:, h] @ kd[h // (heads // kvh)].T / math.sqrt(128)
+        want = torch.softmax(s.masked_fill(~see, -math.inf), -1) @ vd[h // (heads // kvh)]
+        lost += int(want.isnan().any(-1).sum())
+        ok = ~want.isnan()
+        lim = 2e-6 + float(s[s.isfinite()].abs().max()) * 2.0 ** -22
+        for y in (got[:, h], whole[:, h]):
+            assert torch.equal(y.isnan(), want.isnan())
+            assert not ok.any() or float((y - want)[ok].abs().max()) <= lim * float(vd.abs().max())
+    assert lost > 0
+
+
 @pytest.mark.parametrize("scale", [-0.09, 0.0, 3.0])
 @pytest.mark.parametrize("T,start", [(40, 90), (3, 900)])
 def test_attn_prefill_scales(dev, T, start, scale):
