@@ -760,7 +760,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
 
   floatx4 acc[TM][TN];
   int s0[TN];
-  uint32_t lo = 104, hi = 140;
+  uint32_t lo = 103, hi = 140;  // the least scale byte less one (a zero one, which needs no shift, wraps), the largest
 #pragma unroll
   for (int j = 0; j < TN; j++) s0[j] = 0;
   // the lane's operands in a stage: X rows of 16 apart, weight columns of 16 apart
@@ -800,7 +800,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
             const uint32_t e = *(const uint8_t *)(eb + ea + jn * 64);
             sc[jn] = SHIFT ? shifted_scale(e, s0[jn]) : __uint_as_float(e << 23);
             if constexpr (!SHIFT) {
-              lo = min(lo, e);
+              lo = min(lo, e - 1u);
               hi = max(hi, e);
             }
           } else {
@@ -831,8 +831,8 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
   main_loop(std::false_type{});
   bool shift = false;
   if constexpr (MX) {
-    // a scale whose exponent leaves [-23, 13] (or a zero or infinite one): the tile again, its rows shifted
-    if (__ballot(lo < 104 || hi > 140)) shift = true;
+    // a scale whose exponent leaves [-23, 13] (or an infinite one): the tile again, its rows shifted
+    if (__ballot(lo < 103 || hi > 140)) shift = true;
     if (lane == 0) flags[wg] = shift;
   }
   wait_lds();

@@ -4,6 +4,8 @@ dequantize + blocked fp32 GEMM (the reference's shiftScale/Dequantize + sgemm.Mu
 Bar: max|Y - Y_oracle| <= 2e-3 * RMS(Y_oracle) in fp32; the fp16 output equal to RNE of the fp32
 accumulator, bit for bit.
 """
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -195,3 +197,31 @@ def test_mxfp4_gemm_shifted_tiles(dev, orc, m, n, k):
     flat = y.view(-1)
     want16 = ops.silu_mul(flat, flat[1:], "f16", stride=2, n=m * n // 2).view(m, n // 2)
     assert torch.equal(ops.mxfp4_gemm(x, wt, et, "swiglu").view(torch.int16), want16.view(torch.int16))
+
+
+def test_mxfp4_gemm_zero_blocks_run_once(dev):
+    """The encoder gives an all-zero block the scale byte 0, which needs no shift: a product over weights with such a
+    block in every row gives the bits of the same weights with zero codes under an ordinary scale, in the same time
+    (a tile that runs again takes about twice; the bound is halfway)."""
+    m, n, k = 2048, 8192, 2048
+    x = synth.normal(m * k, "k3zero.x").view(m, k)
+    dense = synth.normal(n * k, "k3zero.w", std=0.02, dtype=torch.float32).view(n, k)
+    dense[:, 64:96] = 0
+    w, e = ops.mxfp4_encode(dense)
+    assert int(e[:, 2].max()) == 0 and int(e[:, [0, 1, 3]].min()) > 104
+    plain = e.clone()
+    plain[:, 2] = 120
+    y = [ops.mxfp4_gemm(x, w, s, "f32") for s in (e, plain)]
+    assert torch.equal(y[0].view(torch.int32), y[1].view(torch.int32))
+    best = [math.inf, math.inf]
+    for _ in range(10):
+        for i, s in enumerate((e, plain)):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                ops.mxfp4_gemm(x, w, s, "f32", y=y[0])
+            b.record()
+            b.synchronize()
+            best[i] = min(best[i], a.elapsed_time(b) * 200)
+    print(f"zero blocks {best[0]:.1f} us, none {best[1]:.1f} us", flush=True)
+    assert best[0] <= 1.5 * best[1]
