@@ -397,22 +397,22 @@ __global__ __launch_bounds__(256) void k_attn_prefill_merge(const float *__restr
   const uint32_t cl = min(lane, chunks - 1);
   const float mc = part[cl * kPart + kRows * 128 + rw], lc = part[cl * kPart + kRows * 129 + rw];
   const bool some = lane < chunks && lc != 0.0f;
-  const uint64_t seen = __ballot(some);
   const float top = group_max_dpp<64>(some ? mc : -__builtin_inff());
   const float w = some ? exp2f(mc - top) : 0.0f;
-  const float den = group_sum<64>(some ? w * lc : 0.0f);
+  const float den = group_sum<64>(w * (some ? lc : 0.0f));
+  const int keep = some ? -1 : 0;  // a mask and no selects: the compiler moves loads into a select's branch
   float n0 = 0.0f, n1 = 0.0f;
   for (uint32_t c0 = 0; c0 < chunks; c0 += 8) {
-    float2 o[8];
+    uint2 o[8];
 #pragma unroll
     for (int u = 0; u < 8; u++)
-      o[u] = *(const float2 *)(part + (size_t)min(c0 + u, chunks - 1) * kPart + rw * 128 + 2 * lane);
+      o[u] = *(const uint2 *)(part + (size_t)min(c0 + u, chunks - 1) * kPart + rw * 128 + 2 * lane);
 #pragma unroll
     for (int u = 0; u < 8; u++) {
       const float wc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), (int)(c0 + u)));
-      const bool add = (seen >> (c0 + u)) & 1;  // (c0 + u < 64; lanes past the chunks saw nothing)
-      n0 += add ? wc * o[u].x : 0.0f;
-      n1 += add ? wc * o[u].y : 0.0f;
+      const uint32_t k = (uint32_t)__builtin_amdgcn_readlane(keep, (int)(c0 + u));
+      n0 += wc * __uint_as_float(o[u].x & k);
+      n1 += wc * __uint_as_float(o[u].y & k);
     }
   }
   const size_t o0 = ((size_t)t * a.heads + (h << a.gs) + (row & ((1u << a.gs) - 1))) * 128 + 2 * lane;
