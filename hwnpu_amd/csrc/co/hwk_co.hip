@@ -123,10 +123,16 @@ __device__ __forceinline__ void co_gemm(const uint32_t *X, const uint8_t *W, con
     return;
   }
   const bool equads = MX && (k / 32) % 16 == 0 && ((uintptr_t)E & 15) == 0;
-  // the library's k groups for the shape, so that the sums are its own bit for bit
-  const uint32_t groups = hwk_gemm::pair_takes(MX, m, n, k, E) ? hwk_gemm::pair_groups(MX, m, n, k) : 1;
-  hwk_gemm::gemm_wg<128, 128, MX, 2, 2, 1, true>(blockIdx.x, (const u32x4 *)X, W, E, S, Y, m, n, k, (int)mode, equads,
-                                                 groups);
+  constexpr int kGeneral = 2 * 128 * hwk_gemm::CH, kPair = hwk_gemm::PairCfg<128, 128, MX, 2, 2, 1, 3>::LDS;
+  __shared__ __attribute__((aligned(16))) u32x4 lds[kPair > kGeneral ? kPair : kGeneral];
+  // The paired form in the library's k groups for the shape: its sums bit for bit. Four waves of 64 x 64, a ring of
+  // three stages (MXFP4 512 x 6144 x 2048 30.0 us, 4096 x 8192 x 2048 157; four stages, one workgroup a CU, 36 and
+  // 252; the general form 32 and 190; int8 35.7 and 246, the general form 35.5 and 291).
+  if (hwk_gemm::pair_takes(MX, m, n, k, E))
+    hwk_gemm::gemm_pair_wg<128, 128, MX, 2, 2, 1, 3, true>(blockIdx.x, (const u32x4 *)X, W, E, S, Y, m, n, k, (int)mode,
+                                                           equads, lds, hwk_gemm::pair_groups(MX, m, n, k));
+  else
+    hwk_gemm::gemm_wg<128, 128, MX, 2, 2>(blockIdx.x, (const u32x4 *)X, W, E, S, Y, m, n, k, (int)mode, equads, lds);
 }
 
 __device__ __forceinline__ hwk_moe::MoeArgs moe_args(uint32_t T, uint32_t H, uint32_t I, uint32_t E, uint32_t k,

@@ -11,7 +11,8 @@ template <int BM, int BN, bool MX, int WM, int WN, int KG>
 __global__ __launch_bounds__(64 * WM * WN * KG) __attribute__((amdgpu_waves_per_eu(MX && WM * WN * KG == 4 ? 2 : 1))) void k_gemm(
     const u32x4 *__restrict__ X, const uint8_t *__restrict__ W, const uint8_t *__restrict__ E,
     const uint16_t *__restrict__ S, void *__restrict__ Y, uint32_t M, uint32_t N, uint32_t K, int mode, bool equads) {
-  gemm_wg<BM, BN, MX, WM, WN, KG>(blockIdx.x, X, W, E, S, Y, M, N, K, mode, equads);
+  __shared__ __attribute__((aligned(16))) u32x4 lds[2 * BM * CH];
+  gemm_wg<BM, BN, MX, WM, WN, KG>(blockIdx.x, X, W, E, S, Y, M, N, K, mode, equads, lds);
 }
 
 // Up to 16 waves a CU: as many registers as that leaves a wave.
@@ -19,7 +20,8 @@ template <int BM, int BN, bool MX, int WM, int WN, int KG, int RS, int RES>
 __global__ __launch_bounds__(64 * WM * WN * KG) __attribute__((amdgpu_waves_per_eu(WM * WN * KG * RES / 4))) void k_gemm_pair(
     const u32x4 *__restrict__ X, const uint8_t *__restrict__ W, const uint8_t *__restrict__ E,
     const uint16_t *__restrict__ S, void *__restrict__ Y, uint32_t M, uint32_t N, uint32_t K, int mode, bool equads) {
-  gemm_pair_wg<BM, BN, MX, WM, WN, KG, RS>(blockIdx.x, X, W, E, S, Y, M, N, K, mode, equads);
+  __shared__ __attribute__((aligned(16))) u32x4 lds[PairCfg<BM, BN, MX, WM, WN, KG, RS>::LDS];
+  gemm_pair_wg<BM, BN, MX, WM, WN, KG, RS>(blockIdx.x, X, W, E, S, Y, M, N, K, mode, equads, lds);
 }
 
 // The general form's tile shape for (m, n): the fewest rounds of workgroups over the CUs, a round weighted by the

@@ -65,10 +65,14 @@ __device__ __forceinline__ half8 fp4x8_to_half8(uint32_t w, float s) {
 __device__ __forceinline__ u32x4 load16(const void *p) { return *(const u32x4 *)p; }
 
 // The X chunk (of CH a row a step) that MFMA kk of lane group q reads: the k offsets of a lane's
-// operands in the step. A lane takes 16 values in a row of each 64: values q*16 .. +15 (MFMAs 0, 1) and
-// 64 + q*16 .. +15 (MFMAs 2, 3), of int8 and MXFP4 weights alike. Every form of the GEMM feeds its MFMAs
-// these sets in this order, so that forms and tile shapes agree bit for bit (given the same segments of K).
-__device__ __forceinline__ int xchunk(int q, int kk) { return kk < 2 ? 2 * q + kk : 8 + 2 * q + (kk - 2); }
+// operands in the step. int8: two 16-byte weight loads a lane at q*16 and 64 + q*16 (each 16 rows x 64
+// contiguous bytes a load instruction); MXFP4: one 32-value block a lane at q*32 (one code load and one scale
+// byte: the paired form's order, 16 values of each 64, took two of each and 1.1-1.28 times as long here).
+template <bool MX>
+__device__ __forceinline__ int xchunk(int q, int kk) {
+  if constexpr (MX) return 4 * q + kk;
+  return kk < 2 ? 2 * q + kk : 8 + 2 * q + (kk - 2);
+}
 
 // The first 128-value step of segment g when the S steps of K go to KG segments.
 __host__ __device__ __forceinline__ uint32_t seg_first(uint32_t S, uint32_t KG, uint32_t g) {
@@ -93,7 +97,7 @@ template <int BM, int BN, bool MX, int WM, int WN, int KG>
 struct Stage {
   u32x4 a[Cfg<BM, BN, MX, WM, WN, KG>::AL];
   u32x4 b[Cfg<BM, BN, MX, WM, WN, KG>::TN][Cfg<BM, BN, MX, WM, WN, KG>::BL];
-  uint32_t e[Cfg<BM, BN, MX, WM, WN, KG>::TN][2];  // MXFP4: the scale bytes of the lane's two blocks
+  uint32_t e[Cfg<BM, BN, MX, WM, WN, KG>::TN];  // MXFP4 block scale bytes
   uint32_t k0;                                  // the step's K offset
 };
 
@@ -122,16 +126,12 @@ __device__ __forceinline__ void load_w(Stage<BM, BN, MX, WM, WN, KG> &s, const u
                                        const uint32_t (&brow)[Cfg<BM, BN, MX, WM, WN, KG>::TN], int q, int g) {
   using C = Cfg<BM, BN, MX, WM, WN, KG>;
   if constexpr (MX) {
+    const uint32_t blk = min(k0 + q * 32, K - 32) / 32;
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const uint32_t kc = min(k0 + h * 64 + q * 16, K - 16);
-#pragma unroll
-      for (int j = 0; j < C::TN; j++) {
-        const u32x2 v = *(const u32x2 *)(W + (size_t)brow[j] * (K / 2) + kc / 2);
-        s.b[j][0][2 * h] = v[0];
-        s.b[j][0][2 * h + 1] = v[1];
-        s.e[j][h] = E[(size_t)brow[j] * (K / 32) + kc / 32];
-      }
+    for (int j = 0; j < C::TN; j++) {
+      const size_t bi = (size_t)brow[j] * (K / 32) + blk;
+      s.b[j][0] = load16(W + bi * 16);
+      s.e[j] = E[bi];
     }
   } else {
 #pragma unroll
@@ -154,12 +154,10 @@ __device__ __forceinline__ void zero_tail(Stage<BM, BN, MX, WM, WN, KG> &s, uint
 #pragma unroll
   for (int j = 0; j < C::TN; j++) {
     if constexpr (MX) {
-#pragma unroll
-      for (int h = 0; h < 2; h++)
-        if (s.k0 + h * 64 + q * 16 >= K) {
-          s.b[j][0][2 * h] = s.b[j][0][2 * h + 1] = 0u;
-          s.e[j][h] = 0u;
-        }
+      if (s.k0 + q * 32 >= K) {
+        s.b[j][0] = zero;
+        s.e[j] = 0u;
+      }
     } else {
 #pragma unroll
       for (int h = 0; h < C::BL; h++)
@@ -383,18 +381,102 @@ __device__ __forceinline__ void store_strips(const floatx4 (&acc)[TM][TN], const
   }
 }
 
-// SEG: the accumulators of nseg segments of K (seg_first) are added in order, as the paired form's k groups'
-// are (one segment: the plain sum).
-template <int BM, int BN, bool MX, int WM, int WN, int KG = 1, bool SEG = false>
+// The general form's store through LDS: the wave's whole block (RW x CW) into its region st, the values as
+// store_strips has them, then 16-byte pieces of its rows to Y (in strips the 128 x 128 MXFP4 tile of four waves
+// spills registers). The fp32 rows are padded (P32 = CW + 4 floats) so that the 4 row groups of a write land in
+// different banks (P32 = CW where the padded block does not fit); the fp16 rows are not (padding them measured no
+// faster: their reads of 16 bytes a lane then conflict). For staged(Y, N, mode).
+template <int TM, int TN, int P32>
+struct StageRows {
+  static constexpr int RW = TM * 16, CW = TN * 16;
+  static constexpr int P16 = CW, PH = CW / 2 + 8;  // fp16 rows: full width, SwiGLU half width (padded)
+  static constexpr int FLOATS = RW * P32;              // a region, in floats (the largest of the three)
+  static_assert(P32 == CW || P32 == CW + 4, "fp32 row stride");
+  static_assert(RW * P16 * 2 <= FLOATS * 4 && RW * PH * 2 <= FLOATS * 4, "fp16 rows fit the region");
+};
+template <int BM, int WM, int TM, int TN, bool MX, int P32>
+__device__ __forceinline__ void store_tile_staged(const floatx4 (&acc)[TM][TN], const int (&s0)[TN],
+                                                  const uint16_t *__restrict__ S, void *__restrict__ Y, uint32_t M,
+                                                  uint32_t N, uint32_t m0, uint32_t nw, int wm, int lane, int mode,
+                                                  float *st) {
+  using G = StageRows<TM, TN, P32>;
+  constexpr int RW = G::RW, CW = G::CW;
+  const int r16 = lane & 15, q = lane >> 4;
+  const uint32_t r0 = m0 + wm * RW;
+  auto value = [&](int i, int j, int r) __attribute__((always_inline)) {
+    const float sc = MX ? 1.0f : (float)__builtin_bit_cast(f16, S[min(nw + j * 16 + r16, N - 1)]);
+    return MX ? ldexpf(acc[i][j][r], s0[j]) : acc[i][j][r] * sc;
+  };
+  if (mode == kOutSwiGLU) {
+    // the pairs as store_tile makes them: gate lane rows 0, 1 of its quad, up lane rows 2, 3
+    f16 *h = (f16 *)st;
+    const bool gate = (r16 & 1) == 0;
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = value(i, j, r);
+        const float o0 = __shfl_xor(gate ? v[2] : v[0], 1, 64), o1 = __shfl_xor(gate ? v[3] : v[1], 1, 64);
+        const int row = i * 16 + q * 4 + (gate ? 0 : 2), c = (j * 16 + r16) / 2;
+        h[row * G::PH + c] = (f16)(gate ? swiglu_value(v[0], o0) : swiglu_value(o0, v[2]));
+        h[(row + 1) * G::PH + c] = (f16)(gate ? swiglu_value(v[1], o1) : swiglu_value(o1, v[3]));
+      }
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // this wave's LDS writes done
+    constexpr int CPR = CW / 16;  // 8 outputs a piece
+    for (int c = lane; c < RW * CPR; c += 64) {
+      const int row = c / CPR, k = c % CPR;
+      const uint32_t m = r0 + row, n = nw + k * 16;
+      if (m < M && n < N)
+        *(u32x4 *)((f16 *)Y + (size_t)m * (N / 2) + n / 2) = *(const u32x4 *)(h + row * G::PH + k * 8);
+    }
+  } else if (mode == HWK_OUT_F16) {
+    f16 *h = (f16 *)st;
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) h[(i * 16 + q * 4 + r) * G::P16 + j * 16 + r16] = (f16)f32_value(value(i, j, r));
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+    constexpr int CPR = CW / 8;
+    for (int c = lane; c < RW * CPR; c += 64) {
+      const int row = c / CPR, k = c % CPR;
+      const uint32_t m = r0 + row, n = nw + k * 8;
+      if (m < M && n < N) *(u32x4 *)((f16 *)Y + (size_t)m * N + n) = *(const u32x4 *)(h + row * G::P16 + k * 8);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) st[(i * 16 + q * 4 + r) * P32 + j * 16 + r16] = value(i, j, r);
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+    constexpr int CPR = CW / 4;
+    for (int c = lane; c < RW * CPR; c += 64) {
+      const int row = c / CPR, k = c % CPR;
+      const uint32_t m = r0 + row, n = nw + k * 4;
+      if (m >= M || n >= N) continue;
+      floatx4 v = *(const floatx4 *)(st + row * P32 + k * 4);
+      floatx4 *y = (floatx4 *)((float *)Y + (size_t)m * N + n);
+      if (mode == HWK_OUT_ADD_F32) v = *y + v;
+      *y = v;
+    }
+  }
+}
+
+// lds: 2 * BM * CH 16-byte slots of LDS (the X buffers).
+template <int BM, int BN, bool MX, int WM, int WN, int KG = 1>
 __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X, const uint8_t *__restrict__ W,
                                         const uint8_t *__restrict__ E, const uint16_t *__restrict__ S,
                                         void *__restrict__ Y, uint32_t M, uint32_t N, uint32_t K, int mode,
-                                        bool equads, uint32_t nseg = 1) {
+                                        bool equads, u32x4 *lds) {
   using C = Cfg<BM, BN, MX, WM, WN, KG>;
   constexpr int TM = C::TM, TN = C::TN, NT = C::NT, KKG = C::KKG;
   static_assert(KG == 1 || !MX, "k groups here: int8 only");
   static_assert(KG == 1 || BM * BN * 4 <= 2 * BM * CH * 16, "the k groups' sum goes through the X buffers");
-  __shared__ __attribute__((aligned(16))) u32x4 As[2][BM * CH];
   __shared__ int hs[MX ? BN : 1], ls[MX ? BN : 1];  // the row shift scan (MXFP4)
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int g = wave / (WM * WN), wl = wave % (WM * WN);  // k group, wave in the group
@@ -439,14 +521,6 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int j = 0; j < TN; j++) acc[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
-  floatx4 total[SEG ? TM : 1][SEG ? TN : 1];
-  uint32_t seg = 0;
-  if constexpr (SEG) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) total[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
-  }
 
   // Steps in groups of NS (a partial last group multiplies zeros: its loads read past K). A step:
   // its X slab into LDS, barrier, the next X loads of its stage, then for each kk its weight operands
@@ -457,7 +531,7 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       const uint32_t j = j0 + s;
-      u32x4 *buf = As[s & 1];  // NS is even: step j uses buffer j & 1
+      u32x4 *buf = lds + (s & 1) * (BM * CH);  // NS is even: step j uses buffer j & 1
       if (st[s].k0 + KS > K) zero_tail<BM, BN, MX, WM, WN, KG>(st[s], K, t, q, g);  // uniform: only a ragged step
 #pragma unroll
       for (int i = 0; i < C::AL; i++) {
@@ -468,24 +542,22 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
       issue_order();
       load_x<BM, BN, MX, WM, WN, KG>(st[s], X, M, K, m0, kofs(j + NS), t);
       issue_order();
-      float sc[TN][2];
+      float sc[TN];
 #pragma unroll
-      for (int jn = 0; jn < TN; jn++)
-#pragma unroll
-        for (int h = 0; h < 2; h++) sc[jn][h] = MX ? shifted_scale(st[s].e[jn][h], s0[jn]) : 0.0f;
+      for (int jn = 0; jn < TN; jn++) sc[jn] = MX ? shifted_scale(st[s].e[jn], s0[jn]) : 0.0f;
       // the operands of kk + 1 (X from LDS, weights converted) are fetched before the MFMAs of kk; kk
       // counts the group's MFMAs (the step's MFMA g*KKG + kk)
       auto operands = [&](half8 (&af)[TM], half8 (&bf)[TN], int kk) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < TM; i++) {
           const int row = wm * (BM / WM) + i * 16 + r16;
-          const int ch = KG == 1 ? xchunk(q, kk) : xchunk(q, g * KKG + kk);
+          const int ch = KG == 1 ? xchunk<MX>(q, kk) : xchunk<MX>(q, g * KKG + kk);
           af[i] = __builtin_bit_cast(half8, buf[row * CH + (ch ^ (row & 15))]);
         }
 #pragma unroll
         for (int jn = 0; jn < TN; jn++) {
           if constexpr (MX) {
-            bf[jn] = fp4x8_to_half8(st[s].b[jn][0][kk], sc[jn][kk >> 1]);
+            bf[jn] = fp4x8_to_half8(st[s].b[jn][0][kk], sc[jn]);
           } else {
             const u32x4 v = st[s].b[jn][kk >> 1];  // KG = 2: the group's half, loaded alone
             bf[jn] = i8x8_to_half8(v[(kk & 1) * 2], v[(kk & 1) * 2 + 1]);
@@ -506,28 +578,12 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
       issue_order();
       load_w<BM, BN, MX, WM, WN, KG>(st[s], W, E, K, kofs(j + NS), brow, q, g);
       issue_order();
-      if constexpr (SEG) {
-        for (; seg < nseg && seg_first(steps, nseg, seg + 1) <= j + 1; seg++)  // (empty segments add zeros)
-#pragma unroll
-          for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int jn = 0; jn < TN; jn++) {
-              total[i][jn] += acc[i][jn];
-              acc[i][jn] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
-            }
-      }
     }
-  }
-  if constexpr (SEG) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] = total[i][j];
   }
   if constexpr (KG == 2) {
     // group 1's accumulators to group 0 through the X buffers (every wave is done with them after
     // the barrier), summed in group 0, which writes the tile
-    floatx4 *red = (floatx4 *)&As[0][0];
+    floatx4 *red = (floatx4 *)lds;
     __syncthreads();
     if (g == 1) {
 #pragma unroll
@@ -546,10 +602,13 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
     if (g == 1) return;
   }
   if (staged(Y, N, mode)) {
-    static_assert(WM * WN * 16 * (TN * 16 + 4) * 4 <= 2 * BM * CH * 16, "the store strips fit the X buffers");
+    // a wave's block in region wl of the X buffers (rows padded where that fits)
+    constexpr int CW = TN * 16, PAD = WM * WN * TM * 16 * (CW + 4) <= 2 * BM * CH * 4 ? CW + 4 : CW;
+    using G = StageRows<TM, TN, PAD>;
+    static_assert(WM * WN * G::FLOATS <= 2 * BM * CH * 4, "the staged blocks fit the X buffers");
     if constexpr (KG == 1) __syncthreads();  // every wave is done with the X buffers
-    store_strips<TM, TN, MX>(acc, s0, true, S, Y, M, N, m0 + wm * (BM / WM), nw, lane, mode,
-                             (float *)&As[0][0] + wl * 16 * (TN * 16 + 4));
+    store_tile_staged<BM, WM, TM, TN, MX, PAD>(acc, s0, S, Y, M, N, m0, nw, wm, lane, mode,
+                                               (float *)lds + wl * G::FLOATS);
     return;
   }
   store_tile<BM, WM, TM, TN, MX>(acc, s0, S, Y, M, N, m0, nw, wm, r16, q, mode);
@@ -565,6 +624,9 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
 // A step is one barrier, the operand reads and the MFMAs; nothing is carried in registers but the
 // accumulators, so that a wave fits 128 registers and a CU holds two workgroups: while one waits at its
 // barrier, scans or stores its tile (the SwiGLU's float64 exp), the other's MFMAs run.
+// A lane's operands of a step are the 16 values q*16 .. +15 of a row's 64, in every tile and for both kinds of
+// weights: tiles agree bit for bit given the same segments of K (the code object's kernels, in one tile shape, add
+// the segments that the library's tile has as k groups).
 // The swizzles are applied on the source side (which 16-byte chunk a lane fetches), so that the reads of
 // 16 lanes land in distinct banks:
 //   X   slot p: row p / 8, chunk (p % 8) ^ ((row >> 1) & 7)                (128-byte rows)
@@ -691,14 +753,17 @@ __device__ __forceinline__ bool pair_tile(uint32_t id, uint32_t mt, uint32_t nt,
   return true;
 }
 
-template <int BM, int BN, bool MX, int WM, int WN, int KG, int RS>
+// rings: PairCfg::LDS 16-byte slots of LDS. SEG (one k group, a grid of exactly the tiles, in tile_of's order): the
+// sums of nseg segments of K (seg_first) are added in order, as another tile's k groups' are. (The segment's end is
+// found once a segment: seg_first divides.)
+template <int BM, int BN, bool MX, int WM, int WN, int KG, int RS, bool SEG = false>
 __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restrict__ X, const uint8_t *__restrict__ W,
                                              const uint8_t *__restrict__ E, const uint16_t *__restrict__ S,
                                              void *__restrict__ Y, uint32_t M, uint32_t N, uint32_t K, int mode,
-                                             bool equads) {
+                                             bool equads, u32x4 *rings, uint32_t nseg = 1) {
   using C = PairCfg<BM, BN, MX, WM, WN, KG, RS>;
   constexpr int TM = C::TM, TN = C::TN, NT = C::NT, NW = C::NW, SLOTS = C::SLOTS;
-  __shared__ __attribute__((aligned(16))) u32x4 rings[C::LDS];
+  static_assert(!SEG || KG == 1, "segments in one k group");
   __shared__ uint32_t flags[NW * KG];
   const int t = threadIdx.x, lane = t & 63, wg = __builtin_amdgcn_readfirstlane(t >> 6);
   const int g = wg / NW, wave = wg % NW;  // k group, wave in the group
@@ -706,7 +771,8 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
   const int wm = wave / WN, wn = wave % WN;
   const int r16 = lane & 15, q = lane >> 4;
   uint32_t tm, tn;
-  if (!pair_tile(bx, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn)) return;
+  if constexpr (SEG) tile_of(bx, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn);
+  else if (!pair_tile(bx, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn)) return;
   const uint32_t m0 = tm * BM, n0 = tn * BN;
   const uint32_t nw = n0 + wn * (BN / WN);  // the wave's first column
   // the group's steps of 64 are h0 .. h1-1; all groups run n_steps of them together (a step past a group's
@@ -758,7 +824,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
     else wait_loads<(C::LMIN + 3) * (RS - 2)>();
   };
 
-  floatx4 acc[TM][TN];
+  floatx4 acc[TM][TN], total[SEG ? TM : 1][SEG ? TN : 1];
   int s0[TN];
   uint32_t lo = 103, hi = 140;  // the least scale byte less one (a zero one, which needs no shift, wraps), the largest
 #pragma unroll
@@ -774,6 +840,15 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
     for (int i = 0; i < TM; i++)
 #pragma unroll
       for (int j = 0; j < TN; j++) acc[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t seg = 0, seg_end = 0;  // the segment, the step after its last
+    auto seg_ends = [&](uint32_t g) { return min(2 * seg_first(S128, nseg, g + 1), steps); };
+    if constexpr (SEG) {
+      while ((seg_end = seg_ends(seg)) == 0) seg++;  // (empty ones)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) total[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+    }
 #pragma unroll
     for (int s = 0; s < RS - 1; s++) load(s, s);
     for (uint32_t j0 = 0; j0 < n_steps; j0 += RS) {
@@ -824,9 +899,28 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
             for (int jn = 0; jn < TN; jn++)
               acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[jn], acc[i][jn], 0, 0, 0);
         }
+        if constexpr (SEG) {
+          if (j + 1 == seg_end) {
+            do seg_end = seg_ends(++seg);
+            while (seg < nseg && seg_end == j + 1);  // (empty ones)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+              for (int jn = 0; jn < TN; jn++) {
+                total[i][jn] += acc[i][jn];
+                acc[i][jn] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+              }
+          }
+        }
       }
     }
     wait_loads<0>();  // no load into LDS may land in a stage put to another use
+    if constexpr (SEG) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = total[i][j];
+    }
   };
   main_loop(std::false_type{});
   bool shift = false;

@@ -5,6 +5,7 @@ gfx950 code objects. The GPU half (runs, fences, argument checks on a device) is
 test_runtime_gpu.py."""
 import struct
 
+import msgpack
 import pytest
 
 from hwnpu_amd import hwk
@@ -54,6 +55,18 @@ def test_optional_buffers_from_manifest():
     assert opt["hwk_co_moe_route"] == ["bias"]
     assert opt["hwk_co_moe_gate_up"] == ["gb"] and opt["hwk_co_moe_down"] == ["db"]
     assert all(not v for k, v in opt.items() if "moe" not in k)
+
+
+def test_gemm_kernels_hold_no_scratch():
+    """The metadata of the object's GEMM kernels: no spilled register and no scratch memory (the accumulators and,
+    in the paired form, the segments' sums fill the registers; spilled, a product took three times as long)."""
+    b = image()
+    at = b.index(b"AMDGPU\0")
+    size = struct.unpack("<I", b[at - 8:at - 4])[0]
+    kernels = {k[".name"]: k for k in msgpack.unpackb(b[at + 8:at + 8 + size], strict_map_key=False)["amdhsa.kernels"]}
+    for name in ("hwk_co_mxfp4_gemm", "hwk_co_i8_gemm"):
+        k = kernels[name]
+        assert (k[".vgpr_spill_count"], k[".private_segment_fixed_size"]) == (0, 0), name
 
 
 def test_inspection_module_cannot_run():

@@ -5,6 +5,8 @@ Bar: max|Y - Y_oracle| <= 2e-3 * RMS(Y_oracle) in fp32; the fp16 output equal to
 accumulator, bit for bit.
 """
 import math
+import os
+import re
 
 import numpy as np
 import pytest
@@ -26,8 +28,8 @@ def check_close(got, want, tol=TOL):
     assert err <= tol * rms(want), f"max|d|={err:.4g} rms={rms(want):.4g} ratio={err / rms(want):.3g}"
 
 
-# (512, 6144, 2048) and (500, 6000, 2080) take the 128 x 96 tile of two k groups (the latter with a
-# ragged last step and partial edge tiles); the others the one-group tiles
+# K a multiple of 64: the paired form; (1, 128, 32), (130, 200, 96) and (500, 6000, 2080): the general form, the last
+# in its 128 x 96 tile of two k groups with a ragged last step and partial edge tiles
 @pytest.mark.parametrize("m,n,k", [(512, 6144, 2048), (5, 6144, 2048), (1, 128, 32), (130, 200, 96), (7, 1000, 4096),
                                    (256, 256, 6144), (300, 130, 2880), (500, 6000, 2080)])
 def test_i8_gemm_parity(dev, orc, m, n, k):
@@ -138,26 +140,47 @@ def test_gemm_swiglu_rejects_ragged_n(dev):
         ops.mxfp4_gemm(x, w, e, "swiglu")
 
 
-# One case a tile of the paired form (hwk_gemm's HWK_PAIR_MX / HWK_PAIR_I8, in the tables' order, as pick_pair
-# chooses them), each with rows and columns left over: first with one step of 64 values (fewer than its k
-# groups and ring stages), then with several (a number that its k groups do not divide).
-PAIR_MX = [(898, 6152, 64), (898, 4100, 64), (450, 4100, 64), (289, 4100, 64), (198, 4100, 64), (65, 6152, 64),
-           (37, 4100, 64), (23, 4100, 64), (9, 130, 64)]
-PAIR_I8 = [(898, 4100, 64), (387, 6152, 64), (450, 4100, 64), (198, 4100, 64), (65, 6152, 64), (37, 4100, 64),
-           (23, 4100, 64), (9, 130, 64)]
-PAIR_K = 832
+def _source(name):
+    with open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hwnpu_amd", "csrc", name)) as f:
+        return f.read()
 
 
-@pytest.mark.parametrize("k", [64, 192, PAIR_K])
-@pytest.mark.parametrize("mx,m,n", [(True, m, n) for m, n, _ in PAIR_MX] + [(False, m, n) for m, n, _ in PAIR_I8])
-def test_gemm_paired_tiles(dev, orc, mx, m, n, k):
-    """The paired form's tiles against the oracle in fp32, and their fp16 and added results against their fp32
-    ones bit for bit."""
-    print(f"gemm tiles mx={mx} {m}x{n}x{k}", flush=True)
-    name = f"k3pair.{mx}.{m}.{n}.{k}"
+def paired_tile(mx, m, n, k):
+    """The index of the tile that pick_pair takes, by its rule over the table in gemm_kernels.h."""
+    body = _source("gemm_kernels.h").split("#define HWK_PAIR_" + ("MX" if mx else "I8") + "(F)")[1]
+    body = re.match(r"(?:.*\\\n)*.*\n", body).group(0)
+    best = []
+    for i, t in enumerate(re.findall(r"F\(([\d, ]+)\)", body)):
+        bm, bn, _, _, _, _, res, ps = map(int, t.split(","))
+        most = -(-(-(-m // bm) * -(-n // bn)) // 256)
+        best.append((most * ps * k + -(-most // res) * 3900000, i))
+    return min(best)[1]
+
+
+def general_tile(mx, m, n):
+    """The tile that gemm.hip's pick_shape takes on 256 CUs, by its rule over kShapes."""
+    body = _source("gemm.hip").split("kShapes[] = {")[1].split("};")[0]
+    best = []
+    for t in re.findall(r"\{([\d, ]+)\}", body):
+        bm, bn, wm, wn, kg = map(int, t.split(","))
+        tiles, eight = -(-m // bm) * -(-n // bn), wm * wn * kg == 8
+        if (mx and kg != 1) or (eight and tiles > 256):
+            continue
+        cost = -(-tiles // 256) * bm * bn * (1 + 32 / bm + 32 / bn) * (0.75 if eight else 1)
+        best.append((cost, len(best), (bm, bn, wm, wn, kg)))
+    return min(best)[2]
+
+
+def check_gemm(orc, mx, m, n, k, name, odd_scales=False):
+    """A product against the oracle in fp32, its fp16 and added results against its fp32 ones bit for bit."""
     x = synth.normal(m * k, name + ".x").view(m, k)
     if mx:
         w, e = synth.mxfp4_normal(n, k, name + ".w", std=0.02)
+        if odd_scales:
+            room = torch.empty(e.numel() + 1, dtype=torch.uint8, device="cuda")
+            room[1:] = e.view(-1)
+            e = room[1:].view(e.shape)
+            assert e.data_ptr() % 2 == 1
         wd = orc.mxfp4_dequantize(w.cpu().numpy(), e.cpu().numpy())
         run = lambda mode, y=None: ops.mxfp4_gemm(x, w, e, mode, y=y)  # noqa: E731
     else:
@@ -173,6 +196,46 @@ def test_gemm_paired_tiles(dev, orc, mx, m, n, k):
     b0 = y0.cpu().numpy()
     run("add", y0)
     assert np.array_equal(y0.cpu().numpy(), (b0 + y32).astype(np.float32))
+
+
+# A case for each tile of the paired form (HWK_PAIR_MX, HWK_PAIR_I8, in the tables' order), with rows and columns left
+# over: with one step of 64 values (fewer than its k groups and ring stages), with three (a ring's stages once), and
+# with a number past the ring that its k groups do not divide.
+PAIR_K = 832
+PAIR_MX = [(898, 6152), (898, 4100), (450, 4100), (289, 4100), (198, 4100), (65, 6152), (37, 4100), (23, 4100), (9, 130)]
+PAIR_I8 = [(390, 11044), (387, 6152), (450, 4100), (198, 4100), (65, 6152), (37, 4100), (23, 4100), (9, 130)]
+
+
+@pytest.mark.parametrize("k", [64, 192, PAIR_K])
+@pytest.mark.parametrize("mx,tile,m,n", [(True, i, m, n) for i, (m, n) in enumerate(PAIR_MX)] +
+                         [(False, i, m, n) for i, (m, n) in enumerate(PAIR_I8)] + [(False, None, 898, 4100)])
+def test_gemm_paired_tiles(dev, orc, mx, tile, m, n, k):
+    print(f"gemm tiles mx={mx} tile={tile} {m}x{n}x{k}", flush=True)
+    assert tile is None or paired_tile(mx, m, n, k) == tile
+    check_gemm(orc, mx, m, n, k, f"k3pair.{mx}.{m}.{n}.{k}")
+
+
+# A case for each tile of the general form (kShapes), K 32 past a multiple of 64: three steps of 128 values, the last
+# of 96, and one of 96 alone; rows and columns left over.
+GENERAL = [(True, (128, 64, 2, 4, 1), 33, 100), (True, (64, 128, 2, 2, 1), 146, 8200), (True, (128, 128, 2, 4, 1), 204, 8200),
+           (True, (128, 96, 2, 2, 1), 523, 7212), (True, (128, 64, 2, 2, 1), 668, 5392), (True, (128, 128, 2, 2, 1), 668, 8876),
+           (False, (128, 64, 2, 4, 1), 33, 100), (False, (64, 128, 2, 2, 1), 146, 8200), (False, (128, 96, 2, 2, 2), 204, 8200),
+           (False, (128, 128, 2, 4, 1), 262, 8200), (False, (128, 96, 2, 2, 1), 523, 7212), (False, (128, 64, 2, 2, 1), 668, 5392),
+           (False, (128, 128, 2, 2, 1), 668, 8876)]
+
+
+@pytest.mark.parametrize("k", [96, 352])
+@pytest.mark.parametrize("mx,tile,m,n", GENERAL)
+def test_gemm_general_tiles(dev, orc, mx, tile, m, n, k):
+    print(f"gemm general tiles mx={mx} tile={tile} {m}x{n}x{k}", flush=True)
+    assert general_tile(mx, m, n) == tile
+    check_gemm(orc, mx, m, n, k, f"k3gen.{mx}.{m}.{n}.{k}")
+
+
+@pytest.mark.parametrize("m,n,k", [(37, 200, 128), (300, 130, 832)])
+def test_mxfp4_gemm_odd_scale_address(dev, orc, m, n, k):
+    """Scales that start at an odd address: the general form at a K that the paired one takes otherwise."""
+    check_gemm(orc, True, m, n, k, f"k3odd.{m}.{n}.{k}", odd_scales=True)
 
 
 @pytest.mark.parametrize("m,n,k", [(898, 6144, 64), (450, 4096, 192), (65, 6144, 192), (9, 128, PAIR_K)])

@@ -329,7 +329,8 @@ def test_co_attention_bad_shape_is_nan(device, program):
 
 
 @pytest.mark.parametrize("mx,m,n,k", [(False, 512, 768, 2048), (False, 200, 320, 256), (True, 256, 512, 2048),
-                                      (True, 70, 160, 1056)])
+                                      (True, 70, 160, 1056), (True, 37, 200, 832), (False, 9, 300, 448),
+                                      (True, 130, 260, 64), (False, 300, 320, 352)])
 def test_co_gemm_matches_library(device, program, orc, mx, m, n, k):
     """hwk_co_i8_gemm / hwk_co_mxfp4_gemm against hwk_i8_gemm / hwk_mxfp4_gemm (fp16 out) on the same
     operands, and against the oracle's dequant + fp32 GEMM."""
