@@ -229,14 +229,20 @@ void launch_f16_rows_of(hipStream_t st, const void *w, const void *x, void *y, u
                        (const uint4 *)x, y, n, nc, mode);
 }
 
-// Two rows a wave for 4 vectors and more, once the waves walk several sets (k <= 2048) or a row is several
-// passes: 5 vectors against 16,384 rows of 2,048 17.5 µs (one row a wave: 16.3), 32,768 28.0 (28.2), 151,936 120
-// (132); 4 against 2,048 rows of 8,192 11.6 (10.3), 4,096 16.0 (19.8). Up to 3 vectors the loads bound either
-// (3 against 151,936: 103.6 and 103.8). Four rows a wave hold too many registers (slower than two throughout).
+// Two rows a wave for 4 vectors and more (up to 3 the loads bound either), where that measured no slower than one over
+// k 256..8192 by n 2,048..151,936 (time of two over one):
+//   one pass (k <= 2048): from 32,768 rows, which give every wave several sets (0.69-0.99); 4 or 5 vectors of more than
+//     1,792 values leave one row at its loads' rate, and gain from 131,072 (0.95-0.99; 1.02-1.04 at 32,768)
+//   several, X past 40 KB (fewer than four workgroups a CU): from 4,096 rows (0.65-0.96; 1.1-1.2 at 2,048)
+//   several, X below: up to half a second pass, from 6,000 rows (0.80-0.98; 1.02-1.09 at 4,096); past that 1.0-1.07
+// Four rows a wave hold too many registers (slower than two throughout).
 template <int TT>
 void launch_f16_rows(hipStream_t st, const void *w, const void *x, void *y, uint32_t n, uint32_t nc, int mode) {
   if constexpr (TT >= 4) {
-    if (n >= (nc <= 256 ? 32768u : 4096u)) return launch_f16_rows_of<TT, 2>(st, w, x, y, n, nc, mode);
+    const bool two = nc <= 256              ? n >= (TT < 6 && nc > 224 ? 131072u : 32768u)
+                     : TT * nc * 16 > 40960 ? n >= 4096
+                                            : nc <= 384 && n >= 6000;
+    if (two) return launch_f16_rows_of<TT, 2>(st, w, x, y, n, nc, mode);
   }
   launch_f16_rows_of<TT, 1>(st, w, x, y, n, nc, mode);
 }

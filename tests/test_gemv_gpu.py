@@ -193,9 +193,11 @@ def test_f16_gemv_rows_parity(dev, orc, T, n, k):
 
 
 # two rows a wave: an odd row count (the last set's second row is past the end), a last chunk past the row, rows of
-# several passes, the fewest and the most vectors, and the row counts just below (one row a wave)
+# several passes with X above and below 40 KB, the fewest and the most vectors; and one row a wave just outside each of
+# the rule's lines (the 3rd, 4th, 6th and from the 10th on)
 @pytest.mark.parametrize("T,n,k", [(4, 32769, 512), (8, 32771, 2048), (6, 32767, 264), (4, 4097, 2056), (8, 4096, 4096),
-                                   (5, 4095, 2560), (4, 4099, 8192)])
+                                   (5, 4095, 2560), (4, 4099, 8192), (4, 6001, 2056), (5, 6003, 3072), (5, 5999, 3072),
+                                   (4, 6001, 3080), (4, 32769, 1800), (5, 4097, 4096)])
 @pytest.mark.parametrize("mode", ["f32", "add"])
 def test_f16_gemv_rows_two_a_wave(dev, orc, T, n, k, mode):
     print(f"f16_gemv_rows T={T} n={n} k={k} {mode}", flush=True)
