@@ -925,12 +925,13 @@ namespace {
 
 // The decode-step GEMV's workgroups: 8 waves of 2 rows a pass (x is made once for 8 waves' rows, and
 // the model's shapes still give every CU whole workgroups: qkv 2048 row sets, 256 workgroups;
-// gate_up 6144, 768; measured against 4 and 16 waves, and 4 rows a pass). The merging GEMV takes one row a
-// wave, 256 workgroups for the model's 2,048 rows: with two it leaves half the CUs idle (8 decode steps behind
-// 1,024 positions 5,386 -> 5,341 µs; 16 waves of one row: 5,614).
-template <int BPL, int XM, bool SWIGLU, int MODE>
+// gate_up 6144, 768; measured against 4 and 16 waves, and 4 rows a pass). The merging GEMV takes one row a wave
+// while that is no more than a workgroup a CU (launch_x_bpl): its workgroups each make the merge anew, but two rows
+// a wave leave half the CUs idle (a step of 12 layers at hidden 2048, 219.1 -> 216.9 µs, at 1024, 212.0 -> 209.6; at
+// 2880, past the line, one row takes 255.6 against 241.0, at 8192 with 64 heads 740 against 600).
+template <int BPL, int XM, bool SWIGLU, int MODE, int RPW = 2>
 void launch_x(hipStream_t st, const void *w, const void *e, const XIn &in, void *y, uint32_t n, uint32_t nb) {
-  constexpr int WPB = 8, RPW = XM == X_MERGE && !SWIGLU ? 1 : 2;
+  constexpr int WPB = 8;
   const uint32_t sets = (n + RPW - 1) / RPW;
   const void *xa = XM == X_F16 ? (const void *)in.x16 : XM == X_NORM ? (const void *)in.h : (const void *)in.ws;
 #define HWK_XL(MBC) hipLaunchKernelGGL((k_mxfp4_gemv_x<BPL, RPW, XM, SWIGLU, WPB, MODE, MBC>), dim3((sets + WPB - 1) / WPB), \
@@ -949,6 +950,16 @@ void launch_x(hipStream_t st, const void *w, const void *e, const XIn &in, void 
 
 template <int XM, bool SWIGLU, int MODE>
 void launch_x_bpl(hipStream_t st, const void *w, const void *e, const XIn &in, void *y, uint32_t n, uint32_t nb) {
+  if constexpr (XM == X_MERGE && !SWIGLU) {
+    if (n <= 8 * 256) {
+      switch ((nb + 63) / 64) {
+        case 1: return launch_x<1, XM, SWIGLU, MODE, 1>(st, w, e, in, y, n, nb);
+        case 2: return launch_x<2, XM, SWIGLU, MODE, 1>(st, w, e, in, y, n, nb);
+        case 3: return launch_x<3, XM, SWIGLU, MODE, 1>(st, w, e, in, y, n, nb);
+        default: return launch_x<4, XM, SWIGLU, MODE, 1>(st, w, e, in, y, n, nb);
+      }
+    }
+  }
   switch ((nb + 63) / 64) {
     case 1: launch_x<1, XM, SWIGLU, MODE>(st, w, e, in, y, n, nb); break;
     case 2: launch_x<2, XM, SWIGLU, MODE>(st, w, e, in, y, n, nb); break;

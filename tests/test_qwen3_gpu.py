@@ -78,6 +78,28 @@ def test_qwen3_small_matches_oracle(dev, orc, heads, kv_heads, max_prompt, max_c
     m.close()
 
 
+# past 2,048 rows the step's attention-merging GEMV takes two rows a wave (SMALL's takes one): just past the line, and
+# at the widest heads
+@pytest.mark.parametrize("hidden,heads,kv_heads", [(2080, 16, 8), (4096, 64, 16)])
+def test_qwen3_wider_steps_match_oracle(dev, orc, hidden, heads, kv_heads):
+    cfg = dict(layers=1, hidden=hidden, heads=heads, kv_heads=kv_heads, head_dim=128, inter=512, vocab=1024)
+    print(f"qwen3 wider {cfg}", flush=True)
+    m = Qwen3(**cfg, max_ctx=64, max_prompt=32)
+    m.synth(seed=0, std=0.02)
+    ref = orc.Qwen3(**cfg, max_ctx=64, seed=0, std=0.02)
+    prompt = synth_np.uniform_int(30, 0, cfg["vocab"], "t.qwen3.wider").astype(np.int32)
+    m.prefill(prompt, 0)
+    ref.run(prompt, 0)
+    for i in range(3):  # the device's own token given to the oracle: only the logits are compared
+        tok = int(m.history(30 + i, 1)[0])
+        if i < 2:
+            m.step()
+        else:
+            m.decode(1)
+        check_close(m.logits(), ref.run([tok], 30 + i)[1], f"step {i} logits")
+    m.close()
+
+
 def test_qwen3_rejects_bad_input(dev):
     m = Qwen3(**SMALL, max_ctx=64, max_prompt=32)
     m.synth()
