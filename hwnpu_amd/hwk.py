@@ -177,15 +177,21 @@ class _Lib:
     def __init__(self, path: str):
         self.path = path
         self._cdll = C.CDLL(path)
+        # the ABI first: a library of another one, or an older one of this, may lack entry points
+        try:
+            abi = self._cdll.hwk_abi()
+        except AttributeError:
+            raise HwkLibraryError(f"{path}: no hwk_abi, not libhwk") from None
+        if abi != ABI:
+            raise HwkLibraryError(f"{path}: ABI {abi}, this binding speaks {ABI}")
+        missing = [name for name in SIGNATURES if not hasattr(self._cdll, name)]
+        if missing:
+            raise HwkLibraryError(f"{path}: ABI {abi}, but without {', '.join(missing)}: an older build, build it again")
+        # a checked callable per entry point, made once: made anew at each access they cost more than the call
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(self._cdll, name)
             fn.restype = P if res == ERR else res
             fn.argtypes = args
-        abi = self._cdll.hwk_abi()
-        if abi != ABI:
-            raise HwkLibraryError(f"{path}: ABI {abi}, this binding speaks {ABI}")
-
-        # a checked callable per entry point, made once: made anew at each access they cost more than the call
         for name, (res, _) in SIGNATURES.items():
             fn = getattr(self._cdll, name)
             setattr(self, name, self._checked(name, fn) if res == ERR else fn)

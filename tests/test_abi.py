@@ -1,8 +1,9 @@
-"""libhwk's C ABI on the CPU: it loads, speaks ABI 1, exports every entry point include/hwk.h
+"""libhwk's C ABI on the CPU: it loads, speaks ABI 4, exports every entry point include/hwk.h
 declares, and rejects bad arguments with an error string before any launch. No GPU needed."""
 import ctypes as C
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -48,6 +49,20 @@ def test_wrong_abi_refused(tmp_path, monkeypatch):
     monkeypatch.undo()
     hwk._lib = None
     hwk.load()
+
+
+@pytest.mark.parametrize("source,match", [
+    ("int other(void) { return 0; }", "not libhwk"),
+    ("int hwk_abi(void) { return 3; }", "ABI 3"),
+    ("int hwk_abi(void) { return 4; }", "without hwk_.*older build")])
+def test_older_library_is_refused(tmp_path, monkeypatch, source, match):
+    """A library of another ABI, or an earlier one of this without the newest entry points, is refused by name."""
+    src, lib = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text(source)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    monkeypatch.setattr(hwk, "_lib", None)
+    with pytest.raises(hwk.HwkLibraryError, match=match):
+        hwk.load(str(lib))
 
 
 def test_missing_library_is_loud(tmp_path, monkeypatch):
