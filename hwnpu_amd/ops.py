@@ -24,10 +24,15 @@ def f32_bits(v: float) -> int:
 _U32, _F32 = struct.Struct("<I"), struct.Struct("<f")
 
 
+# the current stream's handle as torch keeps it, where this torch has the call (it is not a public one)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    # the current stream of the current device as torch keeps it; torch.cuda.current_stream() makes a Stream
-    # object for it, 2 µs a call
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    # torch.cuda.current_stream() makes a Stream object for the handle, 2 µs a call
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _need(t: torch.Tensor, name: str, dtype, shape=None):

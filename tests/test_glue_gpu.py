@@ -173,3 +173,16 @@ def test_argmax_ties_and_specials(dev, orc):
     x = np.stack(rows)
     got = ops.argmax(torch.from_numpy(x).cuda()).cpu().numpy().tolist()
     assert got == [orc.argmax(row) for row in rows] == [5, 0, 0, 100, n - 1]
+
+
+@pytest.mark.parametrize("raw", [True, False])
+def test_ops_take_the_current_stream(dev, monkeypatch, raw):
+    """The ops' stream is torch's current one, on a side stream as well, with torch's own call for its handle and
+    without it."""
+    if not raw:
+        monkeypatch.setattr(ops, "_raw_stream", None)
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert ops._stream() == side.cuda_stream
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream != side.cuda_stream
