@@ -1,5 +1,7 @@
 // MoE on gfx950: the kernels of hwk_moe_route, hwk_moe_experts and hwk_moe_layer and their launch
 // choices (the device code is in moe_kernels.h).
+#include <atomic>
+
 #include "hwk_common.h"
 #include "moe_kernels.h"
 
@@ -97,8 +99,19 @@ MoeArgs args_of(const hwk_moe_params *p) {
   return a;
 }
 
+// Allows a kernel its dynamic LDS past 64 KB on the current device (done: the kernel's devices so far, a bit each).
+char *allow_lds(const void *kernel, std::atomic<uint64_t> &done) {
+  int dev = 0;
+  HWK_TRY("hipGetDevice", hipGetDevice(&dev));
+  const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+  if (done.load(std::memory_order_relaxed) & bit) return nullptr;
+  HWK_TRY("hwk_moe (LDS)", hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
+  done.fetch_or(bit, std::memory_order_relaxed);
+  return nullptr;
+}
+
 template <int PPW, bool ROUTE>
-void launch_gate_up(hipStream_t st, const void *x, const float *logits, const float *rbias, int32_t *idx, float *w,
+char *launch_gate_up(hipStream_t st, const void *x, const float *logits, const float *rbias, int32_t *idx, float *w,
                     const void *gu_w, const void *gu_e, const float *gu_b, float *act, MoeArgs a) {
   const uint32_t unique_max = a.T * a.k < a.E ? a.T * a.k : a.E, nb = a.H / 32;
   // tiles a workgroup: one until the grid has twice what the chip holds (four workgroups a CU), then as many as
@@ -108,14 +121,13 @@ void launch_gate_up(hipStream_t st, const void *x, const float *logits, const fl
   a.span = wgs < 2 * goal ? 1 : wgs / goal < kMoeSpan ? wgs / goal : kMoeSpan;
   // with the route folded in, one more column of workgroups: the route's own (moe_gate_up_wg)
   const dim3 g1(gate_up_wgs(a.I, 4 * PPW * a.span) + (ROUTE ? 1 : 0), unique_max);
-  // the attribute: dynamic LDS past 64 KB (8 tokens of H = 8,192 take 128 KB)
+  const uint32_t lds = a.T * x_bytes(a.H);  // 8 tokens of H = 8,192 take 128 KB
 #define HWK_GU(L, B)                                                                                              \
   do {                                                                                                            \
-    static const hipError_t attr = hipFuncSetAttribute((const void *)k_moe_gate_up<L, B, PPW, ROUTE>,             \
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);   \
-    (void)attr;                                                                                                   \
-    hipLaunchKernelGGL((k_moe_gate_up<L, B, PPW, ROUTE>), g1, dim3(256), a.T * x_bytes(a.H), st, (const uint4 *)x, \
-                       logits, rbias, idx, w, (const uint4 *)gu_w, (const uint8_t *)gu_e, gu_b, act, a);          \
+    static std::atomic<uint64_t> done{0};                                                                         \
+    if (lds > 64 * 1024) HWK_Q(allow_lds((const void *)k_moe_gate_up<L, B, PPW, ROUTE>, done));                   \
+    hipLaunchKernelGGL((k_moe_gate_up<L, B, PPW, ROUTE>), g1, dim3(256), lds, st, (const uint4 *)x, logits, rbias, \
+                       idx, w, (const uint4 *)gu_w, (const uint8_t *)gu_e, gu_b, act, a);                         \
   } while (0)
   // lanes a row: 32 up to H = 4,096 (a row sum is then half the steps, and one load takes gate and up)
   if (nb <= 32) HWK_GU(32, 1);
@@ -125,6 +137,7 @@ void launch_gate_up(hipStream_t st, const void *x, const float *logits, const fl
   else if (nb <= 192) HWK_GU(64, 3);
   else HWK_GU(64, 4);
 #undef HWK_GU
+  return nullptr;
 }
 
 // K5b: gate_up (with the route folded in when ROUTE), then down with the ordered combine.
@@ -132,10 +145,8 @@ template <bool ROUTE>
 char *run_experts(hipStream_t st, const void *x, const float *logits, const float *rbias, int32_t *idx, float *w,
                   const void *gu_w, const void *gu_e, const float *gu_b, const void *dn_w, const void *dn_e,
                   const float *dn_b, float *out, float *act, const MoeArgs &a, const char *what) {
-  if (a.T <= 2)
-    launch_gate_up<2, ROUTE>(st, x, logits, rbias, idx, w, gu_w, gu_e, gu_b, act, a);
-  else
-    launch_gate_up<4, ROUTE>(st, x, logits, rbias, idx, w, gu_w, gu_e, gu_b, act, a);
+  if (a.T <= 2) HWK_Q((launch_gate_up<2, ROUTE>(st, x, logits, rbias, idx, w, gu_w, gu_e, gu_b, act, a)));
+  else HWK_Q((launch_gate_up<4, ROUTE>(st, x, logits, rbias, idx, w, gu_w, gu_e, gu_b, act, a)));
   if (char *err = hwk::launched(what)) return err;
   // down: lanes a row by I/32 blocks, the fewest idle slots (8 lanes x 3 blocks for I = 768), and row sets enough
   // that a workgroup has 8 rows to share the staged activations

@@ -117,7 +117,7 @@ def _np(*ts):
 
 @pytest.mark.parametrize("T", [1, 2, 5, 8])
 def test_moe_layer_route_folded(dev, orc, T):
-    """hwk_moe_layer (route folded into the gate_up launch up to 2 tokens, a route launch past that):
+    """hwk_moe_layer (route folded into the gate_up launch up to 5 tokens, a route launch past that):
     idx bit-exact to the oracle's Choose, w within one ulp, the output as hwk_moe_experts' on the
     same choice (and the oracle's)."""
     print(f"moe layer T={T}", flush=True)
@@ -141,8 +141,8 @@ def test_moe_layer_score_collision(dev, orc, T, row):
     the fourth place, expert 5 (logit 0.5) against expert 7 (the next float32 above 0.5): relative to
     the maximum 9 both differences round to -8.5, their scores are equal, and Choose's stable order
     takes the lower index 5 where an order by logit would take 7. The layer (the route folded into
-    gate_up at T = 1, a route launch at T = 5) must use expert 5: idx bit-exact, output as the
-    oracle's."""
+    gate_up, which cannot read this choice off the logits and runs Choose in every workgroup) must use
+    expert 5: idx bit-exact, output as the oracle's."""
     x, logits, gw, ge, dw, de = experts_case(T)
     lg = logits.cpu().numpy()
     lg[row, :] = -5.0
@@ -250,10 +250,13 @@ def test_moe_layer_small_shapes_sigmoid(dev, orc):
         (3, 3, 3, 512, 6112),     # 191 of 192 blocks, every expert by every token
         (1, 2, 1, 96, 8192),      # the longest rows of down
         (8, 64, 8, 1024, 4064),   # several tiles a workgroup of gate_up, the last workgroup's past I
+        (5, 64, 8, 512, 2048),    # several tiles a workgroup, the route folded in
+        (8, 4, 2, 8192, 64),      # 128 KB of x in LDS
+        (5, 4, 2, 8192, 64),      # 80 KB, the route folded in
     ],
 )
 def test_moe_layer_tiles(dev, orc, T, E, k, H, I):
-    """Each layout of gate_up (by H) and of down (by I) at its edges, the route folded in: idx as the
+    """Each layout of gate_up (by H) and of down (by I) at its edges, the route folded in up to 5 tokens: idx as the
     oracle's Choose, the output as the oracle's experts'; hwk_moe_experts with an id out of range and a
     repeated one (neither counts a second time)."""
     print(f"moe layer T={T} E={E} k={k} H={H} I={I}", flush=True)
