@@ -230,7 +230,7 @@ def test_attn_prefill_causal(dev, orc, heads, kvh, T, start, cap):
 
 
 # split over workgroups with a workspace (hwk_attn_prefill_ws): one row, a few, blocks whose last rows are
-# missing, chunks that end inside the causal edge, the most chunks (64); each also without the workspace
+# missing, chunks that end inside the causal edge, many chunks (57); each also without the workspace
 @pytest.mark.parametrize("heads,kvh,T,start,cap", [
     (16, 8, 1, 511, 512), (16, 8, 5, 1024, 1280), (8, 8, 8, 3000, 3072), (32, 8, 33, 1500, 1536), (16, 8, 64, 2000, 2064),
     (32, 8, 130, 4000, 4200), (4, 1, 3, 9000, 9003), (2, 2, 65, 700, 800)])
@@ -257,6 +257,37 @@ def test_attn_prefill_split(dev, orc, heads, kvh, T, start, cap):
         check_close(whole[t], want[t])
     g16 = ops.attn_prefill(q, k, v, start, out_mode="f16").cpu().numpy()
     assert np.array_equal(g16.view(np.uint16), orc.f32_to_f16(got))
+
+
+# one key group a workgroup over many tiles, whose sums go to a second level every 16: 40 tiles unsplit (past 1,536
+# blocks), 23 and 17 tiles a chunk; the most chunks (64); a split prompt from position 0, whose first blocks are one
+# chunk. Scores rise late, far enough that both levels are rescaled after a fold.
+@pytest.mark.parametrize("heads,kvh,T,start,chunks", [(128, 32, 768, 500, 0), (16, 8, 600, 3000, 5), (32, 8, 300, 2300, 5),
+                                                      (4, 1, 3, 10237, 64), (8, 8, 512, 0, 4)])
+def test_attn_prefill_long_chunks(dev, heads, kvh, T, start, chunks):
+    """Sampled rows and heads against float64 softmax; bound as in test_attn_prefill_scales."""
+    from hwnpu_amd import hwk
+
+    print(f"attn prefill long heads={heads} kv={kvh} T={T} start={start}", flush=True)
+    cap, G = start + T, heads // kvh
+    name = f"c3l.{heads}.{T}.{start}"
+    q = synth.normal(T * heads * 128, name + ".q").view(T, heads, 128)
+    k = synth.normal(kvh * cap * 128, name + ".k").view(kvh, cap, 128)
+    v = synth.normal(kvh * cap * 128, name + ".v").view(kvh, cap, 128)
+    k[:, cap * 5 // 8:] *= 4
+    k[:, cap * 7 // 8:] *= 3
+    p = ops.attn_params(heads, kvh, cap, cap)
+    blocks = -(-T * G // 64)
+    assert hwk.load().hwk_attn_prefill_workspace_bytes(T, start, p) == chunks * blocks * kvh * 64 * 130 * 4
+    assert chunks or blocks * kvh >= 1536
+    got = ops.attn_prefill(q, k, v, start, out_mode="f32").cpu()
+    rows = sorted({0, 1, 15, 16, 63, 64, T // 2, T * 7 // 8, T - 2, T - 1} & set(range(T)))
+    see = torch.arange(cap)[None] <= start + torch.tensor(rows)[:, None]
+    for h in sorted({0, 1, heads // 2, heads - 1}):
+        s = q[rows, h].cpu().double() @ k[h // G].cpu().double().T / math.sqrt(128)
+        want = torch.softmax(s.masked_fill(~see, -math.inf), -1) @ v[h // G].cpu().double()
+        lim = 2e-6 + float(s.abs().max()) * 2.0 ** -22
+        assert float((got[rows, h].double() - want).abs().max()) <= lim * float(want.abs().max())
 
 
 def test_attn_prefill_workspace_checked(dev):
