@@ -50,7 +50,6 @@ __device__ __forceinline__ half8 half8_of(u32x4 u) { return __builtin_bit_cast(h
 
 // LDS transpose read: in each 16-lane group, lane 4a + c receives element c of the 8-byte
 // segments addressed by lanes a, a + 4, a + 8, a + 12 of the group.
-typedef __attribute__((address_space(3))) char lds_char;
 __device__ __forceinline__ short4v tr_read(const lds_char *p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)p);
 }
@@ -64,20 +63,6 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
   return d;
 }
-
-// A load of 16 bytes a lane into LDS (lane i at lds + 16 i), in inline assembly so that the compiler adds no
-// wait of its own: the waits below order it (a wave's loads complete in issue order). M0 takes the LDS
-// address, the s_nop is the wait state behind that write.
-__device__ __forceinline__ void to_lds16(const void *sbase, uint32_t voff, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_loads() {  // all but the wave's last N loads done
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
-// A barrier that waits for no memory counter: __syncthreads would wait for the tiles in flight.
-__device__ __forceinline__ void bare_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
 // How a prompt's attention is cut up: blocks of 64 rows a kv head, and chunks of `tiles` key tiles, at most
 // `chunks` a block (1: not split).
@@ -145,7 +130,7 @@ __global__ __launch_bounds__(256 * S) __attribute__((amdgpu_waves_per_eu(3))) vo
   // the group's stages; the lane's loads of a tile: slot p = (i * 4 + wave) * 64 + lane holds chunk p % 16 of
   // key p / 16, swizzled on the source side. Keys past the block's read its last key (masked), tiles past the
   // chunk its last tile.
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char *)lds_all + gi * NST * STAGE;
+  const uint32_t lds0 = lds_at(lds_all) + gi * NST * STAGE;
   constexpr int HALF = LOADS / 2;
   uint32_t lkey[HALF], lk[HALF], lv[HALF];
 #pragma unroll

@@ -291,9 +291,6 @@ __device__ __forceinline__ void store_tile(const floatx4 (&acc)[TM][TN], const i
   }
 }
 
-// LDS writes and reads of this wave done (lgkmcnt 0; the other counters not waited for)
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
-
 // The tile's store through LDS, 16 rows of the wave's block at a time (a strip): the values as stored
 // (fp16 rounded, SwiGLU'd pairs, or scaled fp32), then 16-byte pieces of the rows to Y, since an MFMA
 // tile's lanes hold one column each. Every value is rounded and combined as store_tile does it. st: the
@@ -423,7 +420,7 @@ __device__ __forceinline__ void store_tile_staged(const floatx4 (&acc)[TM][TN], 
         h[row * G::PH + c] = (f16)(gate ? swiglu_value(v[0], o0) : swiglu_value(o0, v[2]));
         h[(row + 1) * G::PH + c] = (f16)(gate ? swiglu_value(v[1], o1) : swiglu_value(o1, v[3]));
       }
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // this wave's LDS writes done
+    wait_lds();
     constexpr int CPR = CW / 16;  // 8 outputs a piece
     for (int c = lane; c < RW * CPR; c += 64) {
       const int row = c / CPR, k = c % CPR;
@@ -439,7 +436,7 @@ __device__ __forceinline__ void store_tile_staged(const floatx4 (&acc)[TM][TN], 
       for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int r = 0; r < 4; r++) h[(i * 16 + q * 4 + r) * G::P16 + j * 16 + r16] = (f16)f32_value(value(i, j, r));
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+    wait_lds();
     constexpr int CPR = CW / 8;
     for (int c = lane; c < RW * CPR; c += 64) {
       const int row = c / CPR, k = c % CPR;
@@ -453,7 +450,7 @@ __device__ __forceinline__ void store_tile_staged(const floatx4 (&acc)[TM][TN], 
       for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int r = 0; r < 4; r++) st[(i * 16 + q * 4 + r) * P32 + j * 16 + r16] = value(i, j, r);
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+    wait_lds();
     constexpr int CPR = CW / 4;
     for (int c = lane; c < RW * CPR; c += 64) {
       const int row = c / CPR, k = c % CPR;
@@ -691,33 +688,6 @@ __host__ __device__ __forceinline__ bool pair_takes(bool mx, uint32_t m, uint32_
          (uint64_t)n * (mx ? k / 2 : k) < (1ull << 32);
 }
 
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-  static_assert(N >= 0 && N <= 63, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-// A workgroup barrier that waits for no memory counter (__syncthreads would wait for every load into
-// LDS in flight, the ring's prefetches included): the caller has waited for its own part.
-__device__ __forceinline__ void ring_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-typedef __attribute__((address_space(3))) void lds_void;
-// The loads into LDS as inline assembly, so that the compiler inserts no wait of its own for them (its
-// wait insertion tracks the LDS targets of a few such loads only, and before an LDS read that none of
-// those covers it waits for every load in flight, which drains the prefetch). The ring's explicit vmcnt
-// waits and barriers order them instead; the "memory" clobber keeps LDS reads and the barriers on their
-// side of each load. The LDS address (wave-uniform) goes in M0 as an operand the compiler sets, the s_nop
-// the wait state between that write and the load; the global address is sbase (scalar) + voff (a lane's
-// offset).
-__device__ __forceinline__ void to_lds16(const void *sbase, uint32_t voff, void *lds) {
-  const uint32_t l = (uint32_t)(uintptr_t)(lds_void *)lds;
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(l) : "memory");
-}
-// 2 bytes a lane, each zero-extended to a dword of LDS
-__device__ __forceinline__ void to_lds2(const void *sbase, uint32_t voff, void *lds) {
-  const uint32_t l = (uint32_t)(uintptr_t)(lds_void *)lds;
-  asm volatile("s_nop 0\n\tglobal_load_lds_ushort %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(l) : "memory");
-}
-
 template <int BM, int BN, bool MX, int WM, int WN, int KG, int RS>
 struct PairCfg {
   static constexpr int NW = WM * WN, NT = 64 * NW * KG;  // waves a group; threads
@@ -805,15 +775,15 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
 #pragma unroll
     for (int a = 0; a < C::AX; a++)
       if (C::XI % NW == 0 || a * NW + wave < C::XI)
-        to_lds16((const char *)X + k0 * 2, xo[a], xb + (a * NW + wave) * 64);
+        to_lds16((const char *)X + k0 * 2, xo[a], lds_at(xb + (a * NW + wave) * 64));
 #pragma unroll
     for (int a = 0; a < C::AW; a++)
       if (C::WI % NW == 0 || a * NW + wave < C::WI)
-        to_lds16((const char *)W + (MX ? k0 / 2 : k0), wo[a], wb + (a * NW + wave) * 64);
+        to_lds16((const char *)W + (MX ? k0 / 2 : k0), wo[a], lds_at(wb + (a * NW + wave) * 64));
 #pragma unroll
     for (int a = 0; a < C::AE; a++)
       if (C::EI % NW == 0 || a * NW + wave < C::EI)
-        to_lds2((const char *)E + k0 / 32, eo[a], eb + (a * NW + wave) * 64);
+        to_lds2((const char *)E + k0 / 32, eo[a], lds_at(eb + (a * NW + wave) * 64));
   };
   // this wave's loads of all steps but the last RS - 2 issued done
   const int extra = (wave < C::XI % NW) + (wave < C::WI % NW) + (wave < C::EI % NW);
@@ -859,7 +829,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
         // every wave's loads of step j landed, every wave done with step j-1's stage, which step j+RS-1 takes
         wait_step();
         wait_lds();
-        ring_barrier();
+        bare_barrier();
         issue_order();
         load(j + RS - 1, (s + RS - 1) % RS);
         issue_order();
@@ -930,7 +900,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
     if (lane == 0) flags[wg] = shift;
   }
   wait_lds();
-  ring_barrier();  // every wave is done with the stages
+  bare_barrier();  // every wave is done with the stages
   if constexpr (MX) {
     shift = false;
 #pragma unroll
@@ -953,7 +923,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
       __syncthreads();
       main_loop(std::true_type{});
       wait_lds();
-      ring_barrier();
+      bare_barrier();
     }
   }
   if constexpr (KG > 1) {
@@ -967,7 +937,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
       for (int j = 0; j < TN; j++) sums[(((g * NW + wave) * TM + i) * TN + j) * 64 + lane] = acc[i][j];
     }
     wait_lds();
-    ring_barrier();
+    bare_barrier();
 #pragma unroll
     for (int i = 0; i < TM; i++) {
       if (i % KG != g) continue;
@@ -983,7 +953,7 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
       }
     }
     wait_lds();
-    ring_barrier();  // the sums are read: the store strips take their place
+    bare_barrier();  // the sums are read: the store strips take their place
   }
   if (staged(Y, N, mode))
     store_strips<TM, TN, MX, KG>(acc, s0, shift, S, Y, M, N, m0 + wm * (BM / WM), nw, lane, mode,

@@ -260,6 +260,36 @@ __device__ __forceinline__ float swiglu_value(float g, float u) {
 // only where a value is used).
 __device__ __forceinline__ void issue_order() { __builtin_amdgcn_sched_barrier(0); }
 
+// ---- loads from memory straight into LDS, and the waits that order them ----
+
+typedef __attribute__((address_space(3))) char lds_char;
+__device__ __forceinline__ uint32_t lds_at(const void *p) { return (uint32_t)(uintptr_t)(lds_char *)p; }
+
+// A load of 16 bytes a lane into LDS (lane i at lds + 16 i), from the scalar base sbase and the lane's byte offset. In
+// inline assembly, so that the compiler inserts no wait of its own for it (its wait insertion tracks the LDS targets
+// of a few such loads only, and before an LDS read that none of those covers it waits for every load in flight, which
+// drains a prefetch): the explicit waits below and barriers order these loads (a wave's complete in issue order), and
+// the "memory" clobber keeps LDS reads and barriers on their side of each. The LDS address (wave-uniform) goes in M0
+// as an operand the compiler sets, the s_nop is the wait state between that write and the load.
+__device__ __forceinline__ void to_lds16(const void *sbase, uint32_t voff, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
+}
+// 2 bytes a lane, each zero-extended to a dword of LDS
+__device__ __forceinline__ void to_lds2(const void *sbase, uint32_t voff, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_ushort %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
+}
+// All but the wave's last N vector loads done (the other counters not waited for).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N >= 0 && N <= 63, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// LDS writes and reads of this wave done (lgkmcnt 0; the other counters not waited for).
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
+// A workgroup barrier that waits for no memory counter (__syncthreads would wait for every load into LDS in flight,
+// the prefetches included): the caller has waited for its own part.
+__device__ __forceinline__ void bare_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
 // Loads the named kernel arguments into SGPRs here, all in one batch with one wait: otherwise the
 // compiler loads each argument where it is first used, and a load issued after an issue_order()
 // fence waits for its argument with a round trip of its own before the global loads behind it issue.

@@ -233,14 +233,6 @@ __device__ __forceinline__ float gated(float g, float u, const MoeArgs &a) {
   return g / (1.0f + (float)exp((double)(-g))) * u;
 }
 
-// A load of 16 bytes a lane into LDS (lane i at lds + 16 i), in inline assembly so that the compiler adds no
-// wait of its own (it would wait for the weights in flight). M0 takes the LDS address, the s_nop is the wait
-// state behind that write.
-typedef __attribute__((address_space(3))) char lds_char;
-__device__ __forceinline__ void to_lds16(const void *sbase, uint32_t voff, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
-}
-
 // A token's x in LDS: whole 1 KB loads, the four 16-byte chunks of block b in the order q ^ (b/4 & 3), so that one
 // chunk of 16 neighbouring blocks fills the banks.
 __host__ __device__ __forceinline__ uint32_t x_bytes(uint32_t H) { return (H * 2 + 1023) / 1024 * 1024; }
@@ -321,7 +313,7 @@ __device__ __forceinline__ void moe_gate_up_wg(uint32_t bx, uint32_t by, const u
   for (uint64_t m = who; m; m &= m - 1)
     if (!slots || (uint32_t)__builtin_ctzll(m) / a.k != (63 - (uint32_t)__builtin_clzll(slots)) / a.k)
       slots |= m & -m;
-  const uint32_t cols = (uint32_t)__builtin_popcountll(slots), xl = (uint32_t)(uintptr_t)(lds_char *)xs;
+  const uint32_t cols = (uint32_t)__builtin_popcountll(slots), xl = lds_at(xs);
   for (uint32_t tile = 0; tile < a.span; tile++) {
     const uint32_t pair0 = ((bx * a.span + tile) * 4 + wave) * PPW;
     // every load issued unconditionally from a clamped row / block (a load under a branch is waited
@@ -349,7 +341,7 @@ __device__ __forceinline__ void moe_gate_up_wg(uint32_t bx, uint32_t by, const u
           to_lds16(x, t * nb * 64 + min(((ch & ~3u) | ((ch ^ ch >> 4) & 3)) * 16, nb * 64 - 16), row + o);
         }
       }
-      __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // the weights and the wave's part of x
+      wait_loads<0>();  // the weights and the wave's part of x
       __syncthreads();
     }
     for (uint32_t col = 0; col < cols; col++) {
@@ -439,7 +431,7 @@ __device__ __forceinline__ void moe_down_wg(uint32_t bx, const float *__restrict
   const uint64_t set = chosen_set(my, n);
   const uint32_t U = (uint32_t)__builtin_popcountll(set);
   const uint32_t row0 = bx * RS;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char *)acts + wave * C::kBufs * C::kActs;
+  const uint32_t lds0 = lds_at(acts) + wave * C::kBufs * C::kActs;
   // the lane's source of load i: unit p = 64 i + lane holds chunk (p % 8) ^ (block & 7) of block p / 8
   auto stage = [&](uint32_t slot, uint32_t buf) __attribute__((always_inline)) {
     const float *src = act + (size_t)slot * a.I;
@@ -471,7 +463,7 @@ __device__ __forceinline__ void moe_down_wg(uint32_t bx, const float *__restrict
     while (who) {
       const uint32_t slot = (uint32_t)__builtin_ctzll(who);
       who &= who - 1;
-      __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // the weights and this slot's activations
+      wait_loads<0>();  // the weights and this slot's activations
       issue_order();
       if (C::kBufs == 2 && who) stage((uint32_t)__builtin_ctzll(who), buf ^ 1);
       const char *av0 = acts + (wave * C::kBufs + buf) * C::kActs;
@@ -497,12 +489,12 @@ __device__ __forceinline__ void moe_down_wg(uint32_t bx, const float *__restrict
         if (l == 0) ys[slot * RS + r * SR + lane / LPR] = y;
       }
       if (C::kBufs == 1 && who) {
-        __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // this slot's reads done
+        wait_lds();  // this slot's reads done
         stage((uint32_t)__builtin_ctzll(who), 0);
       }
       if (C::kBufs == 2) buf ^= 1;
     }
-    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // the reads done before the next expert's loads
+    wait_lds();  // the reads done before the next expert's loads
   }
   if (wave == 0) {
     // the slots of each token by ascending expert id (ids outside [0, E) and repeated ids left out)
