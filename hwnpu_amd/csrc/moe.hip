@@ -149,17 +149,25 @@ char *run_experts(hipStream_t st, const void *x, const float *logits, const floa
   else HWK_Q((launch_gate_up<4, ROUTE>(st, x, logits, rbias, idx, w, gu_w, gu_e, gu_b, act, a)));
   if (char *err = hwk::launched(what)) return err;
   // down: lanes a row by I/32 blocks, the fewest idle slots (8 lanes x 3 blocks for I = 768), and row sets enough
-  // that a workgroup has 8 rows to share the staged activations
+  // that a workgroup has 8 rows to share the staged activations; 2 rows up to H = 512, where 8 leave most CUs idle
+  // (a layer of H = 256, I = 3,200, 1 token: 8.0 µs, with 8 rows 9.6; 8 tokens on 3 experts 34 and 46; at H = 768 2
+  // rows lose, 8 tokens of I = 6,144 0.46 against 0.38 of the time before)
   const uint32_t nbi = a.I / 32;
+  const bool narrow = a.H <= 512;
   if (nbi <= 8) launch_down<8, 1, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 16) launch_down<8, 2, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 24) launch_down<8, 3, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 32) launch_down<16, 2, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 48) launch_down<16, 3, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 64 && narrow) launch_down<32, 2, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 64) launch_down<32, 2, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 96 && narrow) launch_down<32, 3, 1>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 96) launch_down<32, 3, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 128 && narrow) launch_down<64, 2, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 128) launch_down<64, 2, 8>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (nbi <= 192 && narrow) launch_down<64, 3, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else if (nbi <= 192) launch_down<64, 3, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
+  else if (narrow) launch_down<64, 4, 2>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   else launch_down<64, 4, 4>(st, act, idx, w, dn_w, dn_e, dn_b, out, a);
   return hwk::launched(what);
 }

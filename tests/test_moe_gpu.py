@@ -251,6 +251,10 @@ def test_moe_layer_small_shapes_sigmoid(dev, orc):
         (1, 2, 1, 96, 8192),      # the longest rows of down
         (8, 64, 8, 1024, 4064),   # several tiles a workgroup of gate_up, the last workgroup's past I
         (5, 64, 8, 512, 2048),    # several tiles a workgroup, the route folded in
+        (4, 8, 2, 512, 2016),     # two rows a workgroup of down: 32 lanes a row
+        (8, 16, 3, 256, 3008),
+        (3, 3, 3, 544, 6112),     # eight rows a workgroup past that: 64 lanes a row
+        (1, 2, 1, 544, 8192),
         (8, 4, 2, 8192, 64),      # 128 KB of x in LDS
         (5, 4, 2, 8192, 64),      # 80 KB, the route folded in
     ],
