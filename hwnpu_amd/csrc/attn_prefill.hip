@@ -117,14 +117,16 @@ __global__ __launch_bounds__(256 * S) __attribute__((amdgpu_waves_per_eu(3))) vo
   const uint32_t wfull = a.start + p0;  // keys up to here are seen by every row of the wave
   const u32x4 *kh = kc + (size_t)h * a.cap * 16, *vh = vc + (size_t)h * a.cap * 16;
 
-  // the scale's sign (exactly) into q, and a zero scale as q = 0: the scores' largest is then that of the products
-  const uint32_t flip = a.scale_log2 < 0.0f ? 0x80008000u : 0u, keep = a.scale_log2 == 0.0f ? 0u : ~0u;
+  // the scale's sign (exactly) into q, and a zero scale as q times 0 (NaN of a NaN or infinity): the scores' largest
+  // is then that of the products
+  const uint32_t flip = a.scale_log2 < 0.0f ? 0x80008000u : 0u;
+  const f16 unit = (f16)(a.scale_log2 == 0.0f ? 0.0f : 1.0f);
   const float scale = a.scale_log2 == 0.0f ? 1.0f : fabsf(a.scale_log2);
   half8 qv[4];
 #pragma unroll
   for (int s = 0; s < 4; s++) {
     const u32x4 v = qlive ? q[((size_t)tq * a.heads + head) * 16 + s * 4 + grp] : (u32x4){0u, 0u, 0u, 0u};
-    qv[s] = half8_of((v ^ flip) & keep);
+    qv[s] = half8_of(v ^ flip) * unit;
   }
 
   // the group's stages; the lane's loads of a tile: slot p = (i * 4 + wave) * 64 + lane holds chunk p % 16 of

@@ -369,3 +369,20 @@ def test_attn_prefill_scales(dev, T, start, scale):
         want = torch.softmax(s.masked_fill(~see, -math.inf), -1) @ vd[h // 2, :start + T]
         lim = 2e-6 + float(s.abs().max()) * 2.0 ** -22
         assert float((got[:, h] - want).abs().max()) <= lim * float(want.abs().max())
+
+
+@pytest.mark.parametrize("T,start", [(40, 90), (3, 900)])
+def test_attn_prefill_zero_scale_non_finite_query(dev, T, start):
+    """Scale 0 weighs every key alike, but a NaN or infinite value in a query still makes its scores, and its row, NaN."""
+    print(f"attn prefill zero scale, non-finite query T={T} start={start}", flush=True)
+    cap = start + T
+    q = synth.normal(T * 8 * 128, "c3zq.q").view(T, 8, 128)
+    k = synth.normal(4 * cap * 128, "c3zq.k").view(4, cap, 128)
+    v = synth.normal(4 * cap * 128, "c3zq.v").view(4, cap, 128)
+    q[0, 0, 5], q[1, 3, 99], q[T - 1, 7, 64] = math.nan, math.inf, -math.inf
+    bad = torch.zeros(T, 8, dtype=torch.bool)
+    bad[0, 0] = bad[1, 3] = bad[T - 1, 7] = True
+    got = ops.attn_prefill(q, k, v, start, out_mode="f32", scale=0.0).cpu()
+    assert torch.equal(got.isnan(), bad[..., None].expand(T, 8, 128))
+    means = torch.stack([v[:, :start + t + 1].cpu().double().mean(1) for t in range(T)]).repeat_interleave(2, 1)
+    assert float((got.double() - means)[~bad].abs().max()) <= 2e-6 * float(v.abs().max())
