@@ -89,8 +89,8 @@ __host__ __device__ __forceinline__ uint32_t first_block(const PrefillArgs &a, u
 }
 
 // S key groups of four waves: group gi takes the chunk's tiles gi, gi + S, ... with stages of its own; the
-// other groups' (m, l, O^T) then meet the first's in LDS (the Merge rule in base 2).
-template <int S>
+// other groups' (m, l, O^T) then meet the first's in LDS (the Merge rule in base 2). ZERO: the scale is 0.
+template <int S, bool ZERO>
 __global__ __launch_bounds__(256 * S) __attribute__((amdgpu_waves_per_eu(3))) void k_attn_prefill(
     const u32x4 *__restrict__ q, const u32x4 *__restrict__ kc, const u32x4 *__restrict__ vc, void *__restrict__ out,
     float *__restrict__ ws, PrefillArgs a) {
@@ -117,16 +117,17 @@ __global__ __launch_bounds__(256 * S) __attribute__((amdgpu_waves_per_eu(3))) vo
   const uint32_t wfull = a.start + p0;  // keys up to here are seen by every row of the wave
   const u32x4 *kh = kc + (size_t)h * a.cap * 16, *vh = vc + (size_t)h * a.cap * 16;
 
-  // the scale's sign (exactly) into q, and a zero scale as q times 0 (NaN of a NaN or infinity): the scores' largest
-  // is then that of the products
+  // the scale's sign (exactly) into q, and a zero scale as q times 0 (NaN of a NaN or infinity), in a kernel of its own
+  // (in the others its instructions cost 33 rows behind 8,000 keys 18.0 -> 18.7 µs): the scores' largest is then that
+  // of the products
   const uint32_t flip = a.scale_log2 < 0.0f ? 0x80008000u : 0u;
-  const f16 unit = (f16)(a.scale_log2 == 0.0f ? 0.0f : 1.0f);
-  const float scale = a.scale_log2 == 0.0f ? 1.0f : fabsf(a.scale_log2);
+  const float scale = ZERO ? 1.0f : fabsf(a.scale_log2);
   half8 qv[4];
 #pragma unroll
   for (int s = 0; s < 4; s++) {
     const u32x4 v = qlive ? q[((size_t)tq * a.heads + head) * 16 + s * 4 + grp] : (u32x4){0u, 0u, 0u, 0u};
-    qv[s] = half8_of(v ^ flip) * unit;
+    qv[s] = half8_of(v ^ flip);
+    if constexpr (ZERO) qv[s] *= (f16)0.0f;
   }
 
   // the group's stages; the lane's loads of a tile: slot p = (i * 4 + wave) * 64 + lane holds chunk p % 16 of
@@ -437,8 +438,9 @@ char *launch_prefill(hipStream_t st, const void *q, const void *k, const void *v
                      const PrefillArgs &a) {
   uint32_t units = 0;
   for (uint32_t c = 0; c < a.cut.chunks; c++) units += a.cut.blocks - first_block(a, c);
-  hipLaunchKernelGGL((k_attn_prefill<S>), dim3(units * a.kvh), dim3(256 * S), 0, st,
-                     (const u32x4 *)q, (const u32x4 *)k, (const u32x4 *)v, out, ws, a);
+  auto *kernel = a.scale_log2 == 0.0f ? k_attn_prefill<S, true> : k_attn_prefill<S, false>;
+  hipLaunchKernelGGL(kernel, dim3(units * a.kvh), dim3(256 * S), 0, st, (const u32x4 *)q, (const u32x4 *)k,
+                     (const u32x4 *)v, out, ws, a);
   if (char *err = hwk::launched("hwk_attn_prefill")) return err;
   if (a.cut.chunks == 1) return nullptr;
   hipLaunchKernelGGL(k_attn_prefill_merge, dim3(a.cut.blocks * a.kvh * (kRows / 4)), dim3(256), 0, st, ws, out, a);
