@@ -624,13 +624,18 @@ __device__ __forceinline__ void gemm_wg(uint32_t bx, const u32x4 *__restrict__ X
 // A lane's operands of a step are the 16 values q*16 .. +15 of a row's 64, in every tile and for both kinds of
 // weights: tiles agree bit for bit given the same segments of K (the code object's kernels, in one tile shape, add
 // the segments that the library's tile has as k groups).
-// The swizzles are applied on the source side (which 16-byte chunk a lane fetches), so that the reads of
-// 16 lanes land in distinct banks:
-//   X   slot p: row p / 8, chunk (p % 8) ^ ((row >> 1) & 7)                (128-byte rows)
-//   W   int8   slot p: column p / 4, chunk (p % 4) ^ ((column >> 2) & 3)   (64-byte columns)
+// The swizzles are applied on the source side (which 16-byte chunk a lane fetches), so that the lanes of an LDS read
+// that are served at once land in distinct banks. A 16-byte read does not serve 16 neighbouring lanes, but four rows
+// of each quarter of the 16, out of two neighbouring lane groups q, q ^ 1 (what the conflict counter tells: swizzles
+// by row >> 1 and column >> 2, right for 16 neighbours, cost every read twice its cycles). So bit 0 of row >> 1 moves
+// the chunk's bit 1, the one that q ^ 1 flips, and the quarters the other two; int8 columns: the bit that it does not.
+//   X   slot p: row p / 8, chunk (p % 8) ^ x_swizzle(row)                  (128-byte rows)
+//   W   int8   slot p: column p / 4, chunk (p % 4) ^ ((column >> 2) & 2)   (64-byte columns)
 //       MXFP4  slot p: column p / 2, chunk (p % 2) ^ ((column >> 3) & 1)   (32-byte columns)
 //   E   (MXFP4) dword p: column p, the step's two scale bytes
-
+// int8 512 x 6144 x 2048: 2,015,232 -> 49,152 conflict cycles a launch (the rest the store's), 17.06 -> 16.88 us a call; the
+// MXFP4 weights' reads, two 8-byte ones in an instruction, still count four cycles each.
+__device__ __forceinline__ uint32_t x_swizzle(uint32_t row) { return ((row >> 2) & 1) | (row & 2) | ((row >> 1) & 4); }
 
 // A tile of the paired form: BM x BN, WM x WN waves a k group, KG k groups, RS ring stages, the workgroups of
 // it that a CU holds (res), and the picoseconds of a CU that the tile takes a value of K (ps).
@@ -757,13 +762,13 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
   uint32_t xo[C::AX], wo[C::AW], eo[C::AE > 0 ? C::AE : 1];
 #pragma unroll
   for (int a = 0; a < C::AX; a++) {
-    const int p = (a * NW + wave) * 64 + lane, row = p / 8, ch = (p % 8) ^ ((row >> 1) & 7);
+    const int p = (a * NW + wave) * 64 + lane, row = p / 8, ch = (p % 8) ^ x_swizzle(row);
     xo[a] = (min(m0 + row, M - 1) * K + ch * 8) * 2;
   }
 #pragma unroll
   for (int a = 0; a < C::AW; a++) {
     const int p = (a * NW + wave) * 64 + lane, col = p / C::WCH;
-    const int c = (p % C::WCH) ^ (MX ? (col >> 3) & 1 : (col >> 2) & 3);
+    const int c = (p % C::WCH) ^ (MX ? (col >> 3) & 1 : (col >> 2) & 2);
     wo[a] = min(n0 + col, N - 1) * (MX ? K / 2 : K) + c * 16;
   }
 #pragma unroll
@@ -801,8 +806,8 @@ __device__ __forceinline__ void gemm_pair_wg(uint32_t bx, const u32x4 *__restric
   for (int j = 0; j < TN; j++) s0[j] = 0;
   // the lane's operands in a stage: X rows of 16 apart, weight columns of 16 apart
   const uint32_t xa = (wm * (BM / WM) + r16) * 128, wa = (wn * (BN / WN) + r16) * (C::WCH * 16);
-  const uint32_t xsw = (r16 >> 1) & 7;
-  const uint32_t wsl = MX ? (((q >> 1) ^ ((r16 >> 3) & 1)) * 16 + (q & 1) * 8) : (q ^ ((r16 >> 2) & 3)) * 16;
+  const uint32_t xsw = x_swizzle(r16);
+  const uint32_t wsl = MX ? (((q >> 1) ^ ((r16 >> 3) & 1)) * 16 + (q & 1) * 8) : (q ^ ((r16 >> 2) & 2)) * 16;
   const uint32_t ea = (wn * (BN / WN) + r16) * 4 + (q >> 1);
   auto main_loop = [&](auto shifted) __attribute__((always_inline)) {
     constexpr bool SHIFT = decltype(shifted)::value;
