@@ -653,12 +653,12 @@ struct PairTile {
 
 // The tile of least cost for Y (m, n) over k, an index into HWK_PAIR_MX or HWK_PAIR_I8. The cost is that of
 // the busiest of the 256 CUs: ps * k for each of its tiles, and 3.9 us (prologue, the first loads' latency,
-// the groups' sums and the stores) for each round of res tiles. Both constants are fitted to every tile's
-// time on 154 (MXFP4) and 137 (int8) shapes, m 9..8192, n 512..16384, k 512..8192: the tile picked is on
-// average 1 % slower than the best of the table and takes 0.47 (MXFP4) and 0.50 (int8) of the time of the
-// one-workgroup-a-CU tiles of 64..128 rows that stood here before. (int8 128 x 128 in two k groups is set just
-// below the one-group tile, which it beats by 3-7 % when a CU has one tile.) Integer arithmetic, so that
-// the host and a kernel agree.
+// the groups' sums and the stores) for each round of res tiles. Both constants are fitted to the tiles' measured
+// times. Every tile on 224 shapes, m 9..8192, n 512..16384, k 512..8192: the tile picked takes on average 1.011
+// (MXFP4) and 1.005 (int8) of the time of the table's best, 1.22 and 1.26 at most, and 0.58 and 0.60 (most 0.97 and
+// 1.01) of the one-workgroup-a-CU tiles of 64..128 rows that stood here before. (int8 128 x 128 in two k groups is set
+// just below the one-group tile: with one tile a CU it takes 0.94-0.97 of its time from k = 2,048 on, 1.06 at 512.)
+// Integer arithmetic, so that the host and a kernel agree.
 __host__ __device__ __forceinline__ int pick_pair(bool mx, uint32_t m, uint32_t n, uint32_t k) {
 #define HWK_TILE(...) {__VA_ARGS__},
   constexpr PairTile kMx[] = {HWK_PAIR_MX(HWK_TILE)}, kI8[] = {HWK_PAIR_I8(HWK_TILE)};
